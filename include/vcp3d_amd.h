@@ -265,10 +265,13 @@ int vcp_profile_residual(vcp_ctx *ctx, int reps, double ms[2]);
 
 /* Execution option with no counterpart in the reference: the workgroup size
    of the volume kernel (threads per element; 0 restores the default). The
-   sizes available for (nDOFs1D, nInt1D) come from vcp_volume_tiles, the
-   default first; vcp_volume_tiles returns their number. Results of different
-   sizes agree to rounding (the partial sums of the mass-matrix solve are
-   grouped differently); a given size gives identical results every run. */
+   sizes available for (nDOFs1D, nInt1D) come from vcp_volume_tiles, which
+   returns their number. The first is the column kernel (one thread per column
+   of integration points, named by its threads per plane of points), the
+   others are workgroups of that many threads. The default is the column
+   kernel for cases large enough to fill the chip with it and the second size
+   for smaller ones. Results of different sizes agree to rounding (partial sums
+   are grouped differently); a given size gives identical results every run. */
 int vcp_set_tile(vcp_ctx *ctx, int nt);
 
 /* Execution option with no counterpart in the reference (whose only precision

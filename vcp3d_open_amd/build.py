@@ -16,6 +16,8 @@ HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
 SOURCES = ["kernels.hip", "geometry.hip", "setup.cpp", "capi.cpp", "batch.cpp", "contraction_ab.hip"]
 AB_SOURCES = ["contraction_ab.hip"]
+# the column form of the volume kernel, one object per (nDOFs1D, nInt1D)
+SHAPES = [(3, 4), (4, 5), (4, 6), (5, 7), (6, 8), (7, 9)]
 # per-source flags: the device metric terms repeat the host set-up's
 # arithmetic exactly, so neither side contracts multiply-adds
 EXTRA = {"geometry.hip": ["-ffp-contract=off"], "setup.cpp": ["-ffp-contract=off"]}
@@ -28,15 +30,14 @@ COMMON = ["-O3", "-fPIC", "-std=c++17", "--offload-arch=gfx950",
 def build(verbose: bool = False) -> str:
     objdir = os.path.join(HERE, "_build")
     os.makedirs(objdir, exist_ok=True)
-    objs = []
+    units = [(src, os.path.splitext(src)[0] + ".o", EXTRA.get(src, [])) for src in SOURCES]
+    units += [("volume.hip", f"volume_{k}_{m}.o", [f"-DVCP_SHAPE_K={k}", f"-DVCP_SHAPE_M={m}"]) for k, m in SHAPES]
     procs = []
-    for src in SOURCES:
-        obj = os.path.join(objdir, os.path.splitext(src)[0] + ".o")
-        cmd = [HIPCC, *COMMON, *EXTRA.get(src, []), "-x", "hip", "-c", os.path.join(CSRC, src), "-o", obj]
+    for src, obj, flags in units:
+        cmd = [HIPCC, *COMMON, *flags, "-x", "hip", "-c", os.path.join(CSRC, src), "-o", os.path.join(objdir, obj)]
         if verbose:
             print(" ".join(cmd), flush=True)
-        procs.append((src, subprocess.Popen(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)))
-        objs.append(obj)
+        procs.append((obj, subprocess.Popen(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)))
     failed = []
     for src, p in procs:
         out, _ = p.communicate()
@@ -47,9 +48,9 @@ def build(verbose: bool = False) -> str:
             sys.stderr.write(out)
     if failed:
         raise RuntimeError("hipcc failed for " + ", ".join(failed))
-    for lib, srcs in ((LIB, [s for s in SOURCES if s not in AB_SOURCES]), (AB_LIB, AB_SOURCES)):
+    for lib, ab in ((LIB, False), (AB_LIB, True)):
         tmp = lib + ".tmp"
-        objs_l = [os.path.join(objdir, os.path.splitext(s)[0] + ".o") for s in srcs]
+        objs_l = [os.path.join(objdir, obj) for src, obj, _ in units if (src in AB_SOURCES) == ab]
         cmd = [HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", tmp, *objs_l]
         subprocess.run(cmd, check=True)
         os.replace(tmp, lib)

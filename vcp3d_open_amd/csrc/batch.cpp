@@ -30,6 +30,9 @@ struct vcp_batch {
     size_t capCases = 0;
     vcp::WorkItem *dWork = nullptr;
     size_t capWork = 0;
+    vcp::WorkItem *dWorkV = nullptr;   // the items ordered by volume kernel
+    size_t capWorkV = 0;
+    int kind[vcp::kVolKinds + 1] = {}; // first item of each kernel in dWorkV
     int *dStatus = nullptr;
     int nWork = 0;
     int initFrom = -1;                 // cases [initFrom, end) need their first residual
@@ -46,9 +49,10 @@ struct vcp_batch {
     {
       if (dCases) (void) hipFree(dCases);
       if (dWork) (void) hipFree(dWork);
+      if (dWorkV) (void) hipFree(dWorkV);
       if (dStatus) (void) hipFree(dStatus);
-      dCases = nullptr; dWork = nullptr; dStatus = nullptr;
-      capCases = capWork = 0;
+      dCases = nullptr; dWork = nullptr; dWorkV = nullptr; dStatus = nullptr;
+      capCases = capWork = capWorkV = 0;
     }
   };
   hipStream_t stream = nullptr;
@@ -123,8 +127,30 @@ int upload(vcp_batch *b)
     HIP_TRY(grow(&g.dWork, g.capWork, work.size()));
     HIP_TRY(hipMemcpy(g.dCases, tab.data(), tab.size() * sizeof(vcp::CaseDev), hipMemcpyHostToDevice));
     HIP_TRY(hipMemcpy(g.dWork, work.data(), work.size() * sizeof(vcp::WorkItem), hipMemcpyHostToDevice));
+    std::vector<vcp::WorkItem> workV;
+    workV.reserve(work.size());
+    for (int k = 0; k < vcp::kVolKinds; ++k) {
+      g.kind[k] = (int) workV.size();
+      for (size_t ci = 0; ci < g.cases.size(); ++ci)
+        if (vcp::volume_kind(g.cases[ci]->dc, g.nt) == k)
+          workV.insert(workV.end(), work.begin() + g.first[ci], work.begin() + g.first[ci + 1]);
+    }
+    g.kind[vcp::kVolKinds] = (int) workV.size();
+    HIP_TRY(grow(&g.dWorkV, g.capWorkV, workV.size()));
+    HIP_TRY(hipMemcpy(g.dWorkV, workV.data(), workV.size() * sizeof(vcp::WorkItem), hipMemcpyHostToDevice));
   }
   b->dirty = false;
+  return 0;
+}
+
+// Volume launches of a group over its items ordered by the kernel that their
+// cases take, one launch per kernel present.
+int batch_volume(const vcp_batch::Group &g, const vcp::StageCtl &ctl, hipStream_t s)
+{
+  vcp::BatchGroup v = g.view();
+  v.work = g.dWorkV;
+  for (int k = 0; k < vcp::kVolKinds; ++k)
+    HIP_TRY(vcp::launch_batch_volume(v, k, ctl, g.kind[k], g.kind[k + 1] - g.kind[k], s));
   return 0;
 }
 
@@ -139,7 +165,9 @@ int init_pass(vcp_batch *b)
     for (size_t ci = g.initFrom; ci < g.cases.size(); ++ci)
       HIP_TRY(vcp::launch_boundary(g.cases[ci]->dc, b->stream, false));
     HIP_TRY(vcp::launch_batch_faces(v, w0, nw, b->stream));
-    HIP_TRY(vcp::launch_batch_volume(v, kResidualOnly, w0, nw, b->stream));
+    for (size_t ci = g.initFrom; ci < g.cases.size(); ++ci)
+      HIP_TRY(vcp::launch_batch_volume(v, vcp::volume_kind(g.cases[ci]->dc, g.nt), kResidualOnly, g.first[ci],
+                                       g.first[ci + 1] - g.first[ci], b->stream));
     g.initFrom = -1;
   }
   return 0;
@@ -157,7 +185,7 @@ int rk_step(vcp_batch *b)
       const vcp::BatchGroup v = g.view();
       for (vcp_ctx *c : g.cases) HIP_TRY(vcp::launch_boundary(c->dc, b->stream, false));
       HIP_TRY(vcp::launch_batch_faces(v, 0, v.nWork, b->stream));
-      HIP_TRY(vcp::launch_batch_volume(v, *ctl, 0, v.nWork, b->stream));
+      if (int rc = batch_volume(g, *ctl, b->stream)) return rc;
     }
   return 0;
 }
@@ -387,6 +415,7 @@ int vcp_batch_set_tile(vcp_batch *b, int K, int M, int nt)
   HIP_TRY(hipStreamSynchronize(b->stream));
   for (vcp_batch::Group &g : b->groups)
     if (g.K == K && g.M == M) g.nt = nt;
+  b->dirty = true;                     // the items are ordered by volume kernel
   b->drop_graph();
   return 0;
   VCP_GUARD_END
@@ -435,7 +464,7 @@ int vcp_batch_profile(vcp_batch *b, int reps, double *ms, int cap)
       for (vcp_ctx *c : g.cases) HIP_TRY(vcp::launch_boundary(c->dc, b->stream, false));
       HIP_TRY(vcp::launch_batch_faces(v, 0, v.nWork, b->stream));
       HIP_TRY(hipEventRecord(ev[1], b->stream));
-      HIP_TRY(vcp::launch_batch_volume(v, probe, 0, v.nWork, b->stream));
+      if ((rc = batch_volume(g, probe, b->stream))) return rc;
       HIP_TRY(hipEventRecord(ev[2], b->stream));
     }
   HIP_TRY(hipStreamSynchronize(b->stream));

@@ -322,6 +322,7 @@ int vcp_create(const vcp_case_desc *d, const double *elem_grid, vcp_ctx **out)
   }
   for (int q = 0; q < M; ++q) dc.opW[q] = t.w_int[q];
   for (int q = 0; q < K; ++q) dc.opC0[q] = t.c0[q];
+  for (int i = 0; i < M * M; ++i) dc.opDL[i] = t.dLq[i];
   dc.to.w3 = put(t.w3); dc.to.w2 = put(t.w2); dc.to.bc = put(t.basis_center);
   dc.to.P1 = put(t.P1); dc.to.dLq = put(t.dLq); dc.to.Lq = put(t.Lq); dc.to.total = (int) tb.size();
   // open boundaries: face list, own face metric, parameters

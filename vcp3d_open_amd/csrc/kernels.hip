@@ -6,7 +6,9 @@
 //                        per-element face slots (no atomics)
 //   volume_kernel        volume residual, gather of the six face slots,
 //                        per-element entropy mass-matrix PCG, optional
-//                        in-place RK stage update
+//                        in-place RK stage update, one workgroup per element:
+//                        the form of small cases; large ones take the column
+//                        kernel of volume.hip
 //   mach_kernel          boundary-averaged Mach number partial sums (NSCBC)
 //   nscbc_kernel         PC-NSCBC boundary faces: characteristic boundary
 //                        state, polynomial-correction reconstruction, flux
@@ -28,6 +30,7 @@
 //   CG_EntropyVarMassMatrix               CG_MassMatrix.cpp:250-504
 //   ElementClass::ComputeTimeStep         ElementClass.cpp:1522-1644
 //   SolverClass::ExecuteTimeSynchronizationStep  SolverClass.cpp:2177-2422
+#include "device.hpp"
 #include "kernels.hpp"
 
 #include <cstdint>
@@ -45,65 +48,6 @@ namespace {
 enum : int { kBCOutflowNSCBC = 1, kBCInflowStaticNSCBC = 2, kBCInflowTotalNSCBC = 3, kBCInflowSubsonic = 4,
               kBCOutflowSubsonic = 5, kBCWallHeatFlux = 6, kBCWallIsothermal = 7, kBCWallInviscid = 8,
               kBCInflowSupersonic = 9, kBCOutflowSupersonic = 10, kBCFarfield = 11 };
-constexpr double kGam = 1.4;
-constexpr double kGm1 = 0.4;
-constexpr double kPrLam = 0.72;
-constexpr double kPrTurb = 0.90;       // VCP3D_CurviLinear.hpp:176
-constexpr double kLamOverMu = -2.0 / 3.0;
-constexpr double kInvGm1 = 1.0 / kGm1;
-
-// ------------------------------------------------------------ utilities
-constexpr int cmax(int x, int y) { return x > y ? x : y; }
-constexpr int cmin(int x, int y) { return x < y ? x : y; }
-
-__device__ inline double wave_sum(double v)
-{
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-  return v;
-}
-__device__ inline double wave_max(double v)
-{
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v = fmax(v, __shfl_xor(v, off, 64));
-  return v;
-}
-
-// Wave64 reduction through DPP row shifts and row broadcasts (no LDS):
-// sum, or max of non-negative values; lanes without a source contribute 0.
-// The result (lane 63) is returned to every lane.
-template <int CTRL, int ROW_MASK>
-__device__ inline double dpp_f64(double v)
-{
-  const int lo = __double2loint(v), hi = __double2hiint(v);
-  const int rlo = __builtin_amdgcn_update_dpp(0, lo, CTRL, ROW_MASK, 0xf, false);
-  const int rhi = __builtin_amdgcn_update_dpp(0, hi, CTRL, ROW_MASK, 0xf, false);
-  return __hiloint2double(rhi, rlo);
-}
-// Row shift with every row enabled: lanes shifted in from outside the row
-// read 0 (bound_ctrl), so no zeroed destination is needed.
-template <int CTRL>
-__device__ inline double dpp_shr_f64(double v)
-{
-  const int lo = __double2loint(v), hi = __double2hiint(v);
-  const int rlo = __builtin_amdgcn_mov_dpp(lo, CTRL, 0xf, 0xf, true);
-  const int rhi = __builtin_amdgcn_mov_dpp(hi, CTRL, 0xf, 0xf, true);
-  return __hiloint2double(rhi, rlo);
-}
-template <bool MAX>
-__device__ inline double wave_reduce_dpp(double v)
-{
-  auto op = [](double x, double y) { return MAX ? fmax(x, y) : x + y; };
-  v = op(v, dpp_shr_f64<0x111>(v));    // row_shr:1
-  v = op(v, dpp_shr_f64<0x112>(v));    // row_shr:2
-  v = op(v, dpp_shr_f64<0x114>(v));    // row_shr:4
-  v = op(v, dpp_shr_f64<0x118>(v));    // row_shr:8   -> lane 15 of each row: row total
-  v = op(v, dpp_f64<0x142, 0xa>(v));   // row_bcast:15 into rows 1, 3
-  v = op(v, dpp_f64<0x143, 0xc>(v));   // row_bcast:31 into rows 2, 3 -> lane 63: total
-  const int lo = __builtin_amdgcn_readlane(__double2loint(v), 63);
-  const int hi = __builtin_amdgcn_readlane(__double2hiint(v), 63);
-  return __hiloint2double(hi, lo);
-}
 
 // Block reduction with one barrier: partial results go to alternating
 // halves of red (2 * 3 * NT/64 doubles); every half starts at the same offset
@@ -135,81 +79,6 @@ __device__ inline void block_reduce1(double (&v)[NV], double *red, int &half)
     v[q] = s;
   }
   half ^= 1;
-}
-
-// t^(-1/(gamma-1)) = t^(-5/2) for gamma = 1.4, as 1 / (t^2 sqrt(t)).
-__device__ inline double pow_m2p5(double t) { return 1.0 / (t * t * sqrt(t)); }
-
-__device__ inline void ent2prim(const double V[5], double &rho, double &u, double &v, double &w,
-                                double &p, double &eKin)
-{
-  const double V4Inv = 1.0 / V[4];
-  u = -V4Inv * V[1]; v = -V4Inv * V[2]; w = -V4Inv * V[3];
-  eKin = 0.5 * (u * u + v * v + w * w);
-  const double s = kGam - kGm1 * (V[0] - V[4] * eKin);
-  rho = pow_m2p5(-V[4] * exp(s));
-  p = -rho * V4Inv;
-}
-
-
-// Eddy viscosity mu_SGS = rho nu_t of the subgrid scale model at one point,
-// from the velocity gradient G[i][j] = du_i/dx_j and the LES length scale len.
-// WALE (CWALEModel::EddyViscosity, SGSModel.cpp:34-113): with S the
-// symmetric part of G and Sd the traceless symmetric part of G^2,
-// nu_t = (0.325 len)^2 |Sd|^3 / max(|S|^5 + |Sd|^(5/2), 1e-30), |X|^2 = X_ij X_ij.
-// Vreman (CVremanModel::EddyViscosity, :128-210): alpha = G with its trace
-// taken off the diagonal, beta = len^2 alpha alpha^T, B the sum of the
-// principal 2 x 2 minors of beta (clipped at 0),
-// nu_t = 0.07 sqrt(B / max(|alpha|^2, 1e-30)).
-__device__ inline double eddy_viscosity(int model, double len, double rho, const double G[3][3])
-{
-  constexpr double third = 1.0 / 3.0, eps = 1e-30;
-  if (model == kSgsWale) {
-    double G2[3][3];
-#pragma unroll
-    for (int i = 0; i < 3; ++i)
-#pragma unroll
-      for (int j = 0; j < 3; ++j) G2[i][j] = G[i][0] * G[0][j] + G[i][1] * G[1][j] + G[i][2] * G[2][j];
-    const double tr = third * (G2[0][0] + G2[1][1] + G2[2][2]);
-    double s2 = 0.0, sd2 = 0.0;
-#pragma unroll
-    for (int i = 0; i < 3; ++i) {
-      const double d = G2[i][i] - tr;
-      s2 += G[i][i] * G[i][i];
-      sd2 += d * d;
-#pragma unroll
-      for (int j = i + 1; j < 3; ++j) {
-        const double sij = 0.5 * (G[i][j] + G[j][i]), dij = 0.5 * (G2[i][j] + G2[j][i]);
-        s2 += 2.0 * sij * sij;
-        sd2 += 2.0 * dij * dij;
-      }
-    }
-    const double sd32 = sd2 * sqrt(sd2);
-    const double den = s2 * s2 * sqrt(s2) + sqrt(sd32 * sd2);
-    const double l = 0.325 * len;
-    return rho * (l * l) * sd32 / fmax(den, eps);
-  }
-  if (model == kSgsVreman) {
-    const double tr = third * (G[0][0] + G[1][1] + G[2][2]);
-    double al[3][3], a2 = 0.0;
-#pragma unroll
-    for (int i = 0; i < 3; ++i)
-#pragma unroll
-      for (int j = 0; j < 3; ++j) {
-        al[i][j] = i == j ? G[i][j] - tr : G[i][j];
-        a2 += al[i][j] * al[i][j];
-      }
-    const double l2 = len * len;
-    double be[3][3];
-#pragma unroll
-    for (int i = 0; i < 3; ++i)
-#pragma unroll
-      for (int j = i; j < 3; ++j) be[i][j] = l2 * (al[i][0] * al[j][0] + al[i][1] * al[j][1] + al[i][2] * al[j][2]);
-    const double B = be[0][0] * be[1][1] - be[0][1] * be[0][1] + be[0][0] * be[2][2] - be[0][2] * be[0][2]
-                   + be[1][1] * be[2][2] - be[1][2] * be[1][2];
-    return rho * 0.07 * sqrt(fmax(B, 0.0) / fmax(a2, eps));
-  }
-  return 0.0;
 }
 
 // Eddy viscosity at a face point (FluxesFace.cpp:1409-1459, :1481-1494): the
@@ -786,57 +655,6 @@ struct VolArgs {
   double c0[K];                           // phi_q(0): basis at the element centre
   double fvec[4][K];                      // phi(-1), phi(+1), phi'(-1), phi'(+1)
 };
-
-// Characteristic-matching-layer source at one point (ElementClass.cpp:
-// 3887-4117): wave amplitudes of the Cartesian primitive gradients per
-// direction with the outgoing eigenvalues of the layer orientation removed,
-// P = S L mapped to the conservative variables. V: entropy variables,
-// gx/gy/gz their Cartesian gradients, wgt[d] = -J w sigma_d scale_d,
-// nsg[d] the layer orientation. Accumulates into out.
-__device__ __forceinline__ void cml_source(const double V[5], const double gx[5], const double gy[5],
-                                           const double gz[5], const double wgt[3], const double nsg[3],
-                                           double out[5])
-{
-  const double V4Inv = 1.0 / V[4];
-  const double u = -V4Inv * V[1], v = -V4Inv * V[2], w = -V4Inv * V[3];
-  const double ek = 0.5 * (u * u + v * v + w * w);
-  const double s = kGam - kGm1 * (V[0] - V[4] * ek);
-  const double rho = pow_m2p5(-V[4] * exp(s));
-  const double p = -rho * V4Inv, rE = p / kGm1 + rho * ek;
-  const double H = rE / rho - V4Inv, a2 = -kGam * V4Inv, a = sqrt(a2);
-  const double rhoa = rho * a, ovra = 1.0 / rhoa, ova2 = 1.0 / a2, rova = rho / a;
-  const double rhou = rho * u, rhov = rho * v, rhow = rho * w;
-  const double vel[3] = {u, v, w};
-#pragma unroll
-  for (int d = 0; d < 3; ++d) {
-    const double *G = d == 0 ? gx : d == 1 ? gy : gz;
-    double dq[5];
-    dq[0] = rho * G[0] + rhou * G[1] + rhov * G[2] + rhow * G[3] + rE * G[4];
-    dq[1] = -V4Inv * G[1] + (-V4Inv * u) * G[4];
-    dq[2] = -V4Inv * G[2] + (-V4Inv * v) * G[4];
-    dq[3] = -V4Inv * G[3] + (-V4Inv * w) * G[4];
-    dq[4] = p * G[0] + (p * u) * G[1] + (p * v) * G[2] + (p * w) * G[3] + (p * H) * G[4];
-    double l1 = vel[d] - a, l2 = vel[d], l3 = vel[d] + a;
-    if (nsg[d] * l1 > 0.0) l1 = 0.0;
-    if (nsg[d] * l2 > 0.0) l2 = 0.0;
-    if (nsg[d] * l3 > 0.0) l3 = 0.0;
-    const double dun = dq[1 + d];
-    const double La = 0.5 * l1 * (ovra * dq[4] - dun);
-    const double Lb = 0.5 * l3 * (ovra * dq[4] + dun);
-    const double Le = l2 * (dq[0] - ova2 * dq[4]);
-    double P[5];
-    P[0] = rova * (Lb + La) + Le;
-    P[4] = rhoa * (Lb + La);
-#pragma unroll
-    for (int t = 0; t < 3; ++t) P[1 + t] = (t == d) ? (Lb - La) : l2 * dq[1 + t];
-    const double wd = wgt[d];
-    out[0] += wd * P[0];
-    out[1] += wd * (u * P[0] + rho * P[1]);
-    out[2] += wd * (v * P[0] + rho * P[2]);
-    out[3] += wd * (w * P[0] + rho * P[3]);
-    out[4] += wd * (ek * P[0] + rhou * P[1] + rhov * P[2] + rhow * P[3] + P[4] / kGm1);
-  }
-}
 
 // ========================================================== volume kernel
 // One workgroup of NT threads per element. LDS holds the modal state, the
@@ -2733,11 +2551,11 @@ hipError_t boundary_impl(const DeviceCase &dc, hipStream_t s, bool monitor)
   return hipGetLastError();
 }
 
-// Volume workgroup sizes instantiated per (K, M), the default first: the
-// sizes for which the points fit two passes and the DOFs one thread each.
-// The defaults are the autotuner's choices on gfx950 (64 threads at (3, 4)
-// and 128 at (4, 5) run 2.4x and 1.6x faster than 256; the recorded table
-// is vcp3d_open_amd/tiles_gfx950.json).
+// Volume workgroup sizes instantiated per (K, M): first the column kernel,
+// named by the threads of a plane of points (volume.hip), then the sizes of
+// volume_kernel for which the points fit two passes and the modes one thread
+// each, the fastest first.
+#define VCP_COL_TILES(X) X(3, 4, 16) X(4, 5, 32) X(4, 6, 64) X(5, 7, 64) X(6, 8, 64) X(7, 9, 128)
 #define VCP_TILES(X)                                                            \
   X(3, 4, 64) X(3, 4, 128) X(3, 4, 256) X(4, 5, 128) X(4, 5, 256)              \
   X(4, 6, 256) X(4, 6, 128) X(5, 7, 256) X(5, 7, 512) X(6, 8, 256) X(6, 8, 512) \
@@ -2837,6 +2655,7 @@ int volume_tiles(int K, int M, int out[4])
 {
   int n = 0;
 #define X(k, m, nt) if (K == k && M == m && n < 4) out[n++] = nt;
+  VCP_COL_TILES(X)
   VCP_TILES(X)
 #undef X
   return n;
@@ -2847,6 +2666,38 @@ int default_volume_tile(int K, int M)
   int t[4];
   return volume_tiles(K, M, t) > 0 ? t[0] : 0;
 }
+
+// Without a given size, the column kernel where the case has enough elements
+// to fill the chip with it: one wave per element (or several elements per
+// wave) runs longer per element than a workgroup, and 256 CUs hold few of
+// them. Measured on one box, volume launch in us, workgroup / column kernel:
+//   (3, 4) 512 elements 30.4 / 35.8, 1728: 44 / 38, 4096: 78 / 48
+//   (4, 5) 512: 36.8 / 44.5, 1000: 43 / 48, 1728: 72 / 64
+//   (4, 6) 512: 42.3 / 46.9, 1000: 58 / 50
+//   (5, 7) 512: 49.7 / 68.3, 1000: 84 / 84, 1728: 116 / 93
+// With two threads per column (K >= 6 in FP64) the column kernel is ahead
+// from the smallest cases on at (6, 8) (27 elements 93 / 81) and once every CU
+// has one at (7, 9) (64: 87 / 90, 216: 85 / 89, 343: 151 / 110); in the float
+// form from a few hundred ((6, 8) 512: 52 / 70, 1000: 84 / 74; (7, 9) 512: 82 / 86).
+int volume_kind(const DeviceCase &dc, int nt)
+{
+  const int cols = dc.sgs != kSgsNone || dc.nSponge > 0 || dc.fbodyOn ? kVolColsFull : kVolCols;
+  if (nt) return nt == default_volume_tile(dc.K, dc.M) ? cols : kVolWorkgroup;
+  const int least = dc.K <= 5 ? 1024 : dc.mixed ? 640 : dc.K == 6 ? 0 : 257;
+  return dc.nElem >= least ? cols : kVolWorkgroup;
+}
+
+namespace {
+// the workgroup size of volume_kernel: the given one, or the first instantiated
+int workgroup_tile(int K, int M, int nt)
+{
+  if (nt) return nt;
+#define X(k, m, t) if (K == k && M == m && !nt) nt = t;
+  VCP_TILES(X)
+#undef X
+  return nt;
+}
+}  // namespace
 
 hipError_t launch_faces(const DeviceCase &dc, hipStream_t s)
 {
@@ -2866,8 +2717,11 @@ hipError_t launch_boundary(const DeviceCase &dc, hipStream_t s, bool monitor)
 
 hipError_t launch_volume(const DeviceCase &dc, const StageCtl &ctl, hipStream_t s)
 {
-  const int nt = dc.nt ? dc.nt : default_volume_tile(dc.K, dc.M);
+  const int kind = volume_kind(dc, dc.nt), nt = workgroup_tile(dc.K, dc.M, dc.nt);
   const hipError_t e = [&]() -> hipError_t {
+#define X(k, m) if (kind != kVolWorkgroup && dc.K == k && dc.M == m) return volume_cols<k, m>(dc, kind == kVolColsFull, ctl, s);
+    VCP_PAIRS(X)
+#undef X
 #define X(k, m, t) if (dc.K == k && dc.M == m && nt == t) return volume_nt<k, m, t>(dc, ctl, s);
     VCP_TILES(X)
 #undef X
@@ -2990,11 +2844,16 @@ hipError_t launch_batch_faces(const BatchGroup &g, int w0, int nw, hipStream_t s
   return hipErrorInvalidValue;
 }
 
-hipError_t launch_batch_volume(const BatchGroup &g, const StageCtl &ctl, int w0, int nw, hipStream_t s)
+hipError_t launch_batch_volume(const BatchGroup &g, int kind, const StageCtl &ctl, int w0, int nw, hipStream_t s)
 {
   if (nw <= 0) return hipSuccess;
   const DeviceCase &p = *g.proto;
-  const int nt = g.nt ? g.nt : default_volume_tile(p.K, p.M);
+  const int nt = workgroup_tile(p.K, p.M, g.nt);
+#define X(k, m)                                                                                     \
+  if (kind != kVolWorkgroup && p.K == k && p.M == m)                                                \
+    return batch_volume_cols<k, m>(g, kind == kVolColsFull, ctl, w0, nw, s);
+  VCP_PAIRS(X)
+#undef X
 #define X(k, m, t) if (p.K == k && p.M == m && nt == t) return batch_volume_nt<k, m, t>(g, ctl, w0, nw, s);
   VCP_TILES(X)
 #undef X

@@ -60,6 +60,7 @@ struct DeviceCase {
   double opF[4][16] = {};                // phi(-1), phi(+1), phi'(-1), phi'(+1)
   double opW[16] = {};                   // 1D Gauss weights
   double opC0[16] = {};                  // phi_q(0), the basis at the element centre
+  double opDL[96] = {};                  // derivatives of the Gauss points' Lagrange polynomials [point][polynomial]
   double *tables = nullptr;
   double *vgeo = nullptr, *fgeo = nullptr, *econst = nullptr;
   double *vgeoN = nullptr;        // [nElem][kNodalGeo][nDOF] (SGS model only)
@@ -167,6 +168,12 @@ hipError_t launch_faces(const DeviceCase &dc, hipStream_t s);
 // with monitor, also the wall forces into scal[kScalForce ..]
 hipError_t launch_boundary(const DeviceCase &dc, hipStream_t s, bool monitor = false);
 hipError_t launch_volume(const DeviceCase &dc, const StageCtl &ctl, hipStream_t s);
+// the volume kernel with one thread per column of points (volume.hip), one
+// instantiation per supported pair
+template <int K, int M>
+hipError_t volume_cols(const DeviceCase &dc, bool full, const StageCtl &ctl, hipStream_t s);
+template <int K, int M>
+hipError_t batch_volume_cols(const BatchGroup &g, bool full, const StageCtl &ctl, int w0, int nw, hipStream_t s);
 hipError_t launch_time_step(const DeviceCase &dc, hipStream_t s);
 // running averages avg = (1 - factNew) avg + factNew q of the current state
 hipError_t launch_average(const DeviceCase &dc, double factNew, hipStream_t s);
@@ -190,7 +197,13 @@ hipError_t launch_stage0(const DeviceCase &dc, const double *dt, hipStream_t s);
 // Batched launches over the work items [w0, w0 + nw) of a group (cases whose
 // kWordActive word is 0 are skipped).
 hipError_t launch_batch_faces(const BatchGroup &g, int w0, int nw, hipStream_t s);
-hipError_t launch_batch_volume(const BatchGroup &g, const StageCtl &ctl, int w0, int nw, hipStream_t s);
+// kind: volume_kind of every item's case
+hipError_t launch_batch_volume(const BatchGroup &g, int kind, const StageCtl &ctl, int w0, int nw, hipStream_t s);
+// The volume kernel of a case with the given workgroup size (0: the default):
+// volume_kernel, or the column kernel (volume.hip) in its plain form or, for a
+// case with an SGS model, a sponge layer or a body force, its full one.
+enum : int { kVolWorkgroup = 0, kVolCols = 1, kVolColsFull = 2, kVolKinds = 3 };
+int volume_kind(const DeviceCase &dc, int nt);
 // per-element time steps, then per case: the minimum, the synchronization-step
 // clipping into scal[kScalDt], and the step counters; a case with error flags
 // or no steps left is deactivated instead
