@@ -3,6 +3,7 @@
 measurement that bench.py --workload interpolation runs)."""
 from __future__ import annotations
 
+import concurrent.futures
 import os
 import subprocess
 import sys
@@ -16,7 +17,8 @@ HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
 SOURCES = ["kernels.hip", "geometry.hip", "setup.cpp", "capi.cpp", "batch.cpp", "contraction_ab.hip"]
 AB_SOURCES = ["contraction_ab.hip"]
-# the column form of the volume kernel, one object per (nDOFs1D, nInt1D)
+# compiled once per shape (nDOFs1D, nInt1D)
+SHAPE_SOURCES = ["volume.hip", "volume_workgroup.hip", "face.hip"]
 SHAPES = [(3, 4), (4, 5), (4, 6), (5, 7), (6, 8), (7, 9)]
 # per-source flags: the device metric terms repeat the host set-up's
 # arithmetic exactly, so neither side contracts multiply-adds
@@ -31,21 +33,25 @@ def build(verbose: bool = False) -> str:
     objdir = os.path.join(HERE, "_build")
     os.makedirs(objdir, exist_ok=True)
     units = [(src, os.path.splitext(src)[0] + ".o", EXTRA.get(src, [])) for src in SOURCES]
-    units += [("volume.hip", f"volume_{k}_{m}.o", [f"-DVCP_SHAPE_K={k}", f"-DVCP_SHAPE_M={m}"]) for k, m in SHAPES]
-    procs = []
-    for src, obj, flags in units:
+    units += [(src, f"{os.path.splitext(src)[0]}_{k}_{m}.o", [f"-DVCP_SHAPE_K={k}", f"-DVCP_SHAPE_M={m}"])
+              for src in SHAPE_SOURCES for k, m in SHAPES]
+
+    def compile_unit(unit):
+        src, obj, flags = unit
         cmd = [HIPCC, *COMMON, *flags, "-x", "hip", "-c", os.path.join(CSRC, src), "-o", os.path.join(objdir, obj)]
         if verbose:
             print(" ".join(cmd), flush=True)
-        procs.append((obj, subprocess.Popen(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)))
+        return subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+
     failed = []
-    for src, p in procs:
-        out, _ = p.communicate()
-        if p.returncode != 0:
-            failed.append(src)
-            sys.stderr.write(out)
-        elif verbose and out.strip():
-            sys.stderr.write(out)
+    jobs = min(8, os.cpu_count() or 1)
+    with concurrent.futures.ThreadPoolExecutor(jobs) as pool:
+        for (src, obj, _), p in zip(units, pool.map(compile_unit, units)):
+            if p.returncode != 0:
+                failed.append(obj)
+                sys.stderr.write(p.stdout)
+            elif verbose and p.stdout.strip():
+                sys.stderr.write(p.stdout)
     if failed:
         raise RuntimeError("hipcc failed for " + ", ".join(failed))
     for lib, ab in ((LIB, False), (AB_LIB, True)):

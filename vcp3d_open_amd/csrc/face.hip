@@ -1,0 +1,527 @@
+// Interior (and periodic) face residuals (gfx950). Compiled once per shape
+// (VCP_SHAPE_K, VCP_SHAPE_M).
+//
+// Reference behaviour followed (VCP3D_CurviLinear/src/):
+//   ElementClass::{I,J,K}FaceResiduals    ElementClass.cpp:2582-3400
+//   FluxesInternalFace / InviscidFluxesFace / ViscousFluxesFace /
+//   PenAndSymFluxesSymmVar                FluxesFace.cpp:220-343, :813-975,
+//                                         :1290-1651, :1152-1284
+#include "device.hpp"
+#include "kernels.hpp"
+#include "transforms.hpp"
+
+namespace vcp {
+namespace {
+
+template <int K, int M, typename T = double>
+struct FaceOps {
+  EvenOdd<K, M, T> a;          // phi_q(r_p) and phi'_q(r_p), even-odd form
+  EvenOddD<K, M, T> d;
+  T A[M * K], D[M * K];        // the same, row-major (p, q)
+  T F[4][K];                   // phi(-1), phi(+1), phi'(-1), phi'(+1)
+  double w[M];                 // 1D Gauss weights
+  double c03;                  // phi_0^3, the value of the constant mode
+};
+
+// Face kernel arguments: the case part (single-case launch) or the case
+// table and work items (batched launch), and the operators (the
+// metric-indexing mode is the kernel's BUG parameter).
+template <int K, int M, typename T = double>
+struct FaceArgs {
+  CaseDev c;
+  const CaseDev *cases;
+  const WorkItem *work;
+  int w0, n;                   // first work item (batch), number of elements
+  FaceOps<K, M, T> op;
+};
+
+// ============================================================ face kernel
+// Faces in direction DIR: each lane group of a wave (the wave, or 32 or 16
+// lanes where the M^2 points fill only that many) takes one element's min
+// face. Side 0 is the element itself (its min face), side 1 the neighbour L
+// (its max face); the normal points from L to the element. When the fast
+// contraction (2 * 5 K columns) and the points (M^2) fit the wave, those
+// phases overwrite their own input in place (every line is read before any is
+// stored); otherwise (K = 7, M = 9) T gets a region of its own. LDS regions:
+//   X: normal contraction B -> fast contraction T -> flux and Cartesian
+//      symmetrising fluxes at the points (over B, or over T when in place)
+//   Y: the first lift stage of one side: flux + fast slot of five variables,
+//      slow slot and normal slot of variables 1..4
+//
+// What bounds it: instruction issue and latency at three waves per SIMD (LDS),
+// not memory. The line contractions use the even-odd operators, the lift
+// fills the wave (9 M lines per side), the pointwise fluxes take five
+// reciprocals and roots instead of twenty divisions and square roots, and two
+// or four faces share a wave at M = 5 and 4: 1520 vector instructions per
+// face instead of 2070 at (5, 7). Measured, launch over the three directions
+// of a Taylor-Green case before / after, us: (3, 4) 18^3 72 / 43,
+// (4, 5) 16^3 68 / 48, (4, 6) 14^3 54 / 46, (5, 7) 32^3 612 / 530,
+// (6, 8) 16^3 194 / 133, (7, 9) 14^3 232 / 214; mixed (3, 4) 71 / 34,
+// (5, 7) 498 / 437.
+template <int K, int M, typename T = double>
+struct FaceSmem {
+  // faces per wave and lanes per face: the pointwise fluxes are half of the
+  // instructions, and the M^2 points of one face leave most of a wave idle at
+  // M = 4 and 5 ((3, 4) 18^3: 57 us with one face per wave, 43 with four)
+  static constexpr int NF = M * M <= 16 ? 4 : M * M <= 32 ? 2 : 1, G = 64 / NF;
+  static constexpr bool kInPlace = 2 * 5 * K <= 64 && M * M <= 64;
+  // traces: the value of five variables, the fast and normal derivatives of
+  // variables 1..4 (the fluxes need no gradient of the first); points: the
+  // flux of five variables, the symmetrising fluxes of 1..4 (the first's are 0)
+  static constexpr int kB = 2 * 2 * 5 * K * K, kT1 = 13 * K * M, kT = 2 * kT1, kP = 17 * M * M;
+  static constexpr int kOffT = kInPlace ? 0 : cmax(kB, kP);   // the fluxes start at 0
+  static constexpr int kX = kInPlace ? cmax(cmax(kB, kT), kP) : kOffT + kT;
+  static constexpr int kY = 13 * M * K;
+  static constexpr int kBytes = (int) sizeof(T) * (2 * M * K + 4 * K + NF * (kX + kY)) + 8 * (M * M + NF * 82);
+  // waves per SIMD to compile for: three when 12 faces fit a CU's 160 KB
+#ifndef VCP_F32_FACE_WAVES
+#define VCP_F32_FACE_WAVES 3
+#endif
+  static constexpr int kWaves = sizeof(T) == 4 && 4 * VCP_F32_FACE_WAVES * kBytes <= 160 * 1024 ? VCP_F32_FACE_WAVES
+                                : 12 * kBytes <= 160 * 1024 ? 3 : 2;
+  T A[M * K], D[M * K];
+  double W2[M * M];
+  T F[4][K];                       // phi(-1), phi(+1), phi'(-1), phi'(+1)
+  struct Face {
+    double Cm[2][4][9];            // metric of points 1..4 (bug)
+    double Mean[2][5];             // float form: mode 0 of both elements
+    T X[kX];
+    T Y[kY];
+  } f[NF];
+};
+
+// args: the kernel's argument block, read in place from the kernel-argument
+// segment by both forms, so that run-time-indexed operator rows come through
+// scalar loads and the single-case and batched kernels do the same
+// arithmetic. T: the type of the contractions (double, or float for the
+// mixed-precision form, where the traces carry the variation about each
+// element's mean, added back at the points in double, and the pointwise
+// fluxes stay in double). SGS: the case has a subgrid scale model (a
+// separate instantiation: its eddy-viscosity code raises the register peak).
+template <int K, int M, int DIR, bool BUG, bool BATCH, typename T, bool SGS>
+__device__ __forceinline__ void face_body(const FaceArgs<K, M, T> &args, const CaseDev a, FaceSmem<K, M, T> &sm,
+                                          int e, bool live)
+{
+#define VCP_FOPS (args.op)
+  constexpr bool kMixed = sizeof(T) == 4;
+  // the element below; a physical boundary face is left to the boundary kernels
+  int L = a.nbr[e * 6 + 2 * DIR];
+  live = live && L >= 0;
+  if (!__any(live)) return;
+  if (L < 0) L = e;
+  constexpr int ND = K * K * K, N2 = M * M;
+  using S = FaceSmem<K, M, T>;
+  constexpr int G = S::G;
+  // strides of the (normal, fast, slow) axes in the [k][j][i] DOF layout
+  constexpr int SN = DIR == 0 ? 1 : DIR == 1 ? K : K * K;
+  constexpr int SFA = DIR == 0 ? K : 1;
+  constexpr int SSL = DIR == 2 ? K : K * K;
+  // parametric slot of each axis: r = 0, s = 1, t = 2 -> (normal, fast, slow)
+  constexpr int PN = DIR, PF = DIR == 0 ? 1 : 0, PS = DIR == 2 ? 1 : 2;
+  T *sA = sm.A, *sD = sm.D;
+  double *sW2 = sm.W2;
+  const int lane = threadIdx.x, tid = lane % G;   // lane of the wave, of the face
+  typename S::Face &sf = sm.f[lane / G];
+  T *B = sf.X;                                // [side][value|deriv][5][K][K]
+  T *Tb = sf.X + S::kOffT;                    // [side][A|D|N][5, 4, 4][K][M]
+  T *sFlux = sf.X, *sFC = sf.X + 5 * N2;      // flux [5][N2], Cartesian sym [x|y|z][4][N2] of variables 1..4
+  // operators in LDS: read as wave-uniform LDS operands in the contractions
+  // (as kernel arguments they would not fit the scalar registers)
+  for (int i = lane; i < M * K; i += 64) { sA[i] = VCP_FOPS.A[i]; sD[i] = VCP_FOPS.D[i]; }
+  for (int i = lane; i < 4 * K; i += 64) sm.F[i / K][i % K] = VCP_FOPS.F[i / K][i % K];
+  // operators of the line contractions, through scalar loads
+  auto ops = [&]() { auto p = (cptr<FaceOps<K, M, T>>) (uintptr_t) &args.op; asm volatile("" : "+s"(p)); return p; };
+  for (int i = lane; i < N2; i += 64) sW2[i] = VCP_FOPS.w[i % M] * VCP_FOPS.w[i / M];
+  const double *g = a.fgeo + ((size_t) e * 3 + DIR) * kFaceGeo * N2;
+  // Loads issued here and used after the contractions, so that their latency
+  // passes under them: the two length scales and, when the points fit the
+  // wave in one pass, this lane's point metric (normal, area and, unless the
+  // metric comes from sm.Cm, both sides' inverse metric).
+  const double lenE = a.econst[(size_t) e * kElemConst + DIR], lenL = a.econst[(size_t) L * kElemConst + DIR];
+  constexpr bool kGeoEarly = N2 <= G;
+  double geoCm[2][9], geoN[4];
+  if constexpr (kGeoEarly) {
+    const int mm = tid < N2 ? tid : 0;
+    if constexpr (!BUG)
+#pragma unroll
+      for (int q = 0; q < 9; ++q) { geoCm[0][q] = g[(13 + q) * N2 + mm]; geoCm[1][q] = g[(4 + q) * N2 + mm]; }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) geoN[q] = g[q * N2 + mm];
+  }
+  if constexpr (BUG)
+#pragma unroll
+    for (int it = 0; it < (72 + G - 1) / G; ++it) {
+      const int i = tid + G * it;
+      if (i < 72) {
+        const int side = i / 36, l = (i / 9) % 4, q = i % 9;
+        sf.Cm[side][l][q] = g[(side ? 4 + q : 13 + q) * N2 + 1 + l];
+      }
+    }
+  if constexpr (kMixed)
+    if (tid < 10) sf.Mean[tid / 5][tid % 5] = a.U[(size_t) (tid < 5 ? e : L) * 5 * ND + (tid % 5) * ND];
+  group_sync<64>();
+  // normal contraction straight from HBM: B[side][0|1][v][s][f]; the loads of
+  // both sides (K <= 6, at most 40 registers) or of one side at a time (K = 7)
+  // are issued before the first of them is waited for. In the float form the
+  // mean (mode 0) is added at the points.
+  constexpr int NIT = (5 * K * K + G - 1) / G;
+  constexpr int SB = 2 * NIT * K <= 40 ? 2 : 1;
+#pragma unroll
+  for (int s0 = 0; s0 < 2; s0 += SB) {
+    double xu[SB][NIT][K];
+#pragma unroll
+    for (int sb = 0; sb < SB; ++sb) {
+      const double *Us = a.U + (size_t) (s0 + sb ? L : e) * 5 * ND;
+#pragma unroll
+      for (int it = 0; it < NIT; ++it) {
+        const int pc0 = tid + G * it, pc = pc0 < 5 * K * K ? pc0 : 0;
+        const int v = pc / (K * K), sl = (pc / K) % K, f = pc % K;
+        const double *u = Us + v * ND + sl * SSL + f * SFA;
+#pragma unroll
+        for (int t = 0; t < K; ++t) xu[sb][it][t] = u[t * SN];
+      }
+    }
+#pragma unroll
+    for (int sb = 0; sb < SB; ++sb) {
+      const int side = s0 + sb;
+      const T *Fv = sm.F[side], *dFv = sm.F[2 + side];
+#pragma unroll
+      for (int it = 0; it < NIT; ++it) {
+        const int pc = tid + G * it;
+        if (pc < 5 * K * K) {
+          const int sl = (pc / K) % K, f = pc % K;
+          T b0 = 0, b1 = 0;
+#pragma unroll
+          for (int t = 0; t < K; ++t) {
+            const T x = (kMixed && t == 0 && sl == 0 && f == 0) ? T(0) : T(xu[sb][it][t]);
+            b0 += Fv[t] * x; b1 += dFv[t] * x;
+          }
+          B[(side * 2 + 0) * 5 * K * K + pc] = b0;
+          B[(side * 2 + 1) * 5 * K * K + pc] = b1;
+        }
+      }
+    }
+  }
+  group_sync<64>();
+  // fast tangential contraction (in place over B when single-pass):
+  // T[side][A|D|N][v][s][f'], f' < M
+  constexpr int RF = (2 * 5 * K + G - 1) / G;
+  T in[S::kInPlace ? RF : 1][2][K];
+  auto read_line = [&](int r, T (&x)[2][K]) {
+    const int c = tid + r * G;
+    if (c < 2 * 5 * K) {
+      const int side = c / (5 * K), vs = c - side * 5 * K;
+#pragma unroll
+      for (int f = 0; f < K; ++f) {
+        x[0][f] = B[(side * 2 + 0) * 5 * K * K + vs * K + f];
+        x[1][f] = B[(side * 2 + 1) * 5 * K * K + vs * K + f];
+      }
+    }
+  };
+  if constexpr (S::kInPlace) {
+#pragma unroll
+    for (int r = 0; r < RF; ++r) read_line(r, in[r]);
+    group_sync<64>();
+  }
+#pragma unroll
+  for (int r = 0; r < RF; ++r) {
+    T (&x)[2][K] = in[S::kInPlace ? r : 0];
+    if constexpr (!S::kInPlace) read_line(r, x);
+    const int c = tid + r * G;
+    if (c >= 2 * 5 * K) continue;
+    const int side = c / (5 * K), vs = c - side * 5 * K;
+    // [A: 5 variables][D: 4][N: 4][s][f'], D and N of variables 1..4
+    T *Ts = Tb + side * S::kT1 + vs * M;
+    const auto op = ops();
+    const EvenOdd<K, M, T> A = scalar_op<K, M, T>(&op->a);
+    T tA[M], tD[M], tN[M];
+    to_points(A, x[0], tA);
+    to_points(A, x[1], tN);
+    to_points(scalar_op<K, M, T>(&op->d), x[0], tD);
+#pragma unroll
+    for (int n = 0; n < M; ++n) Ts[n] = tA[n];
+    if (vs >= K)
+#pragma unroll
+      for (int n = 0; n < M; ++n) { Ts[4 * K * M + n] = tD[n]; Ts[8 * K * M + n] = tN[n]; }
+  }
+  group_sync<64>();
+  // per point: traces, averaged Cartesian gradients of the entropy variables
+  // and the fluxes (Ismail-Roe, viscous, penalty, symmetrising); the outputs
+  // overwrite T in place when single-pass, else the dead B
+  const double lenScale = fmin(lenE, lenL);
+  const double tau = a.tauFact / lenScale;
+  // LES length scale of the face: the mean of the two elements'
+  // (ElementClass.cpp:2655)
+  const double lenLES = SGS ? 0.5 * (a.econst[(size_t) e * kElemConst + kElemLenLES]
+                                     + a.econst[(size_t) L * kElemConst + kElemLenLES]) : 0.0;
+  double evMax = 0.0;
+  for (int m0 = 0; m0 < N2; m0 += G) {
+    const int m = m0 + tid;
+    if (m >= N2) break;
+    const int sp = m / M, fp = m - sp * M;
+    T ai[K], di[K];
+#pragma unroll
+    for (int sl = 0; sl < K; ++sl) { ai[sl] = sA[sp * K + sl]; di[sl] = sD[sp * K + sl]; }
+    double Vs[2][5], gx[5], gy[5], gz[5];
+#pragma unroll
+    for (int v = 0; v < 5; ++v) { gx[v] = 0.0; gy[v] = 0.0; gz[v] = 0.0; }
+#pragma unroll
+    for (int side = 0; side < 2; ++side) {
+      double cm[9];
+      if constexpr (!BUG) {
+#pragma unroll
+        for (int q = 0; q < 9; ++q) cm[q] = kGeoEarly ? geoCm[side][q] : g[(side ? 4 + q : 13 + q) * N2 + m];
+      }
+#pragma unroll
+      for (int v = 0; v < 5; ++v) {
+        const T *tA = Tb + side * S::kT1 + v * K * M + fp;
+        const T *tD = tA + 4 * K * M, *tN = tA + 8 * K * M;
+        T val = 0, gN = 0, gF = 0, gS = 0;
+#pragma unroll
+        for (int sl = 0; sl < K; ++sl) {
+          const T xa = tA[sl * M];
+          val += ai[sl] * xa;
+          if (v > 0) { gS += di[sl] * xa; gN += ai[sl] * tN[sl * M]; gF += ai[sl] * tD[sl * M]; }
+        }
+        Vs[side][v] = kMixed ? double(val) + VCP_FOPS.c03 * sf.Mean[side][v] : double(val);
+        if (v == 0) continue;
+        const double gr = DIR == 0 ? gN : gF;
+        const double gs = DIR == 0 ? gF : DIR == 1 ? gN : gS;
+        const double gt = DIR == 2 ? gN : gS;
+        const double *c = cm;
+        if constexpr (BUG) c = sf.Cm[side][v - 1];
+        gx[v] += 0.5 * (gr * c[0] + gs * c[3] + gt * c[6]);
+        gy[v] += 0.5 * (gr * c[1] + gs * c[4] + gt * c[7]);
+        gz[v] += 0.5 * (gr * c[2] + gs * c[5] + gt * c[8]);
+      }
+    }
+    // materialise the traces and gradients here: otherwise the compiler sinks
+    // their computation into the flux and keeps the LDS operands live
+#pragma unroll
+    for (int v = 0; v < 5; ++v) asm volatile("" : "+v"(Vs[0][v]), "+v"(Vs[1][v]));
+#pragma unroll
+    for (int v = 1; v < 5; ++v) asm volatile("" : "+v"(gx[v]), "+v"(gy[v]), "+v"(gz[v]));
+    const double nn[3] = {kGeoEarly ? geoN[0] : g[0 * N2 + m], kGeoEarly ? geoN[1] : g[1 * N2 + m],
+                          kGeoEarly ? geoN[2] : g[2 * N2 + m]};
+    const double wA = sW2[m] * (kGeoEarly ? geoN[3] : g[3 * N2 + m]);
+    double fl[5], FX[5], FY[5], FZ[5], ev = 0.0;
+    if constexpr (SGS) {
+      ev = face_eddy(a.sgs, lenLES, Vs[1], Vs[0], gx, gy, gz);
+      evMax = fmax(evMax, ev);
+    }
+    point_flux(Vs[1], Vs[0], gx, gy, gz, nn, wA, tau, a.mu, a.thetaHalf, fl, FX, FY, FZ, 1.0, false, 0.0, nullptr,
+               SGS, ev);
+#pragma unroll
+    for (int v = 0; v < 5; ++v) {
+      sFlux[v * N2 + m] = T(fl[v]);
+      if (v > 0) {
+        sFC[(v - 1) * N2 + m] = T(FX[v]); sFC[(3 + v) * N2 + m] = T(FY[v]); sFC[(7 + v) * N2 + m] = T(FZ[v]);
+      }
+    }
+  }
+  if (SGS && a.eddyPart) {
+    // the face's eddy-viscosity maximum for the monitoring data
+    // (FluxesFace.cpp:336-342)
+    evMax = lanes_reduce<G, true>(evMax);
+    if (tid == 0 && live) a.eddyPart[a.nElem + 3 * e + DIR] = evMax;
+  }
+  group_sync<64>();
+  // ---- lift, one side at a time. Fast-axis lines into Y: the flux (with A)
+  // plus the fast slot (with D) of five variables, and the slow and the normal
+  // slot (with A) of variables 1..4; with one face per wave and 9 M <= 64 both
+  // kinds of lines share a pass. Then the slow axis, straight into the face
+  // slot of that side: the value plane (A of the first, D of the slow slot)
+  // and the normal-derivative plane (A of the normal slot) [0|1][v][slow]
+  // [fast]; the volume kernel applies the face vectors.
+  constexpr bool kShare = S::NF == 1 && 9 * M <= 64;
+  static_assert(4 * K <= G || S::NF == 1, "the derivative plane's lines in one pass");
+#pragma unroll
+  for (int side = 0; side < 2; ++side) {
+    const T sign = side ? T(1) : T(-1);
+    double *out = a.faceRes + ((size_t) (side ? L : e) * 6 + 2 * DIR + side) * 10 * K * K;
+    T *Y0 = sf.Y, *YS = sf.Y + 5 * M * K, *YN = YS + 4 * M * K;
+    // Cartesian symmetrising flux mapped to this side's parametric slot P
+    auto coef = [&](int v, int m, int P, int x) {
+      return BUG ? sf.Cm[side][v][3 * P + x] : g[(side ? 4 + 3 * P + x : 13 + 3 * P + x) * N2 + m];
+    };
+    // lines [0, 5 M): flux and fast slot; [5 M, 9 M): slow and normal slot
+    auto lines = [&](int item, bool first, bool second, bool isSecond) {
+      const int idx = isSecond ? item - 5 * M : item;
+      const int v = isSecond ? 1 + idx / M : idx / M, sp = idx % M;
+      const int vc = v > 0 ? v - 1 : 0, P0 = isSecond ? PN : PF;
+      double cb[3], ca[3];
+      if constexpr (BUG)
+#pragma unroll
+        for (int x = 0; x < 3; ++x) { cb[x] = coef(vc, 0, P0, x); ca[x] = coef(vc, 0, PS, x); }
+      T xa[M], xb[M];
+#pragma unroll
+      for (int q = 0; q < M; ++q) {
+        const int m = sp * M + q;
+        const double fx = sFC[vc * N2 + m], fy = sFC[(4 + vc) * N2 + m], fz = sFC[(8 + vc) * N2 + m];
+        if constexpr (!BUG)
+#pragma unroll
+          for (int x = 0; x < 3; ++x) { cb[x] = coef(vc, m, P0, x); ca[x] = coef(vc, m, PS, x); }
+        xb[q] = !isSecond && v == 0 ? T(0) : T(fx * cb[0] + fy * cb[1] + fz * cb[2]);
+        if (!second) xa[q] = sign * sFlux[v * N2 + m];
+        else if (!first) xa[q] = T(fx * ca[0] + fy * ca[1] + fz * ca[2]);
+        else xa[q] = isSecond ? T(fx * ca[0] + fy * ca[1] + fz * ca[2]) : sign * sFlux[v * N2 + m];
+      }
+      const auto op = ops();
+      const EvenOdd<K, M, T> A = scalar_op<K, M, T>(&op->a);
+      T u[K], w[K], z[K];
+      to_modes(A, xa, u);
+      if (second) to_modes(A, xb, w);
+      if (first) {
+#pragma unroll
+        for (int n = 0; n < K; ++n) z[n] = u[n];
+        add_modes(scalar_op<K, M, T>(&op->d), xb, z);
+        if (!isSecond)
+#pragma unroll
+          for (int n = 0; n < K; ++n) Y0[idx * K + n] = z[n];
+      }
+      if (second && isSecond)
+#pragma unroll
+        for (int n = 0; n < K; ++n) { YS[idx * K + n] = u[n]; YN[idx * K + n] = w[n]; }
+    };
+    if constexpr (kShare) {
+      if (tid < 9 * M) lines(tid, true, true, tid >= 5 * M);
+    } else {
+#pragma unroll
+      for (int r = 0; r < (5 * M + G - 1) / G; ++r)
+        if (tid + r * G < 5 * M) lines(tid + r * G, true, false, false);
+#pragma unroll
+      for (int r = 0; r < (4 * M + G - 1) / G; ++r)
+        if (tid + r * G < 4 * M) lines(5 * M + tid + r * G, false, true, true);
+    }
+    group_sync<64>();
+    // slow-axis lines [0, 5 K) of the value plane, [5 K, 9 K) of the derivative plane
+    auto planes = [&](int item, bool first, bool deriv) {
+      const int idx = deriv ? item - 5 * K : item, v = deriv ? 1 + idx / K : idx / K, f = idx % K;
+      const T *ya = deriv ? YN + (v - 1) * M * K + f : Y0 + v * M * K + f;
+      const T *yb = YS + (v > 0 ? v - 1 : 0) * M * K + f;
+      const bool slow = !deriv && v > 0;
+      T xa[M], xb[M], u[K];
+#pragma unroll
+      for (int q = 0; q < M; ++q) { xa[q] = ya[q * K]; xb[q] = first && slow ? yb[q * K] : T(0); }
+      const auto op = ops();
+      to_modes(scalar_op<K, M, T>(&op->a), xa, u);
+      if (first) add_modes(scalar_op<K, M, T>(&op->d), xb, u);
+      if (!live) return;
+      double *o = out + (deriv ? 5 * K * K : 0) + v * K * K + f;
+#pragma unroll
+      for (int n = 0; n < K; ++n) o[n * K] = double(u[n]);
+      if (first && item < K)
+#pragma unroll
+        for (int n = 0; n < K; ++n) out[5 * K * K + n * K + f] = 0.0;
+    };
+    if constexpr (S::NF == 1) {
+      static_assert(9 * K <= 64, "the slow-axis lines in one pass");
+      if (tid < 9 * K) planes(tid, true, tid >= 5 * K);
+    } else {
+#pragma unroll
+      for (int r = 0; r < (5 * K + G - 1) / G; ++r)
+        if (tid + r * G < 5 * K) planes(tid + r * G, true, false);
+      if (tid < 4 * K) planes(5 * K + tid, false, true);
+    }
+    group_sync<64>();
+  }
+#undef VCP_FOPS
+}
+
+// The three directions in one launch: blockIdx.y is the direction;
+// blockIdx.x the element, or (BATCH) a work item (case, element) of the
+// group. The argument block is read through the kernel-argument segment
+// pointer: a by-value copy indexed at run time would go to scratch. The SGS
+// form is compiled for two waves per SIMD, where its eddy-viscosity code fits
+// the registers without spilling.
+template <int K, int M, bool BUG, bool BATCH, typename T, bool SGS>
+__global__ __launch_bounds__(64, (SGS ? cmin(2, FaceSmem<K, M, T>::kWaves) : FaceSmem<K, M, T>::kWaves))
+void face_kernel(FaceArgs<K, M, T> a_)
+{
+  __shared__ FaceSmem<K, M, T> sm;
+  (void) a_;
+  const FaceArgs<K, M, T> &a = *(const FaceArgs<K, M, T> *) __builtin_amdgcn_kernarg_segment_ptr();
+  using S = FaceSmem<K, M, T>;
+  const int sub = threadIdx.x / S::G, item = blockIdx.x * S::NF + sub;
+  bool live = S::NF == 1 || item < a.n;
+  CaseDev c;
+  int e;
+  if constexpr (BATCH) {
+    const WorkItem w = a.work[a.w0 + (live ? item : 0)];
+    c = a.cases[w.c];
+    e = w.e;
+    live = live && c.flags[kWordActive] != 0;
+    if (!__any(live)) return;
+  } else {
+    c = a.c;
+    e = live ? item : 0;
+  }
+  if (blockIdx.y == 0) face_body<K, M, 0, BUG, BATCH, T, SGS>(a, c, sm, e, live);
+  else if (blockIdx.y == 1) face_body<K, M, 1, BUG, BATCH, T, SGS>(a, c, sm, e, live);
+  else face_body<K, M, 2, BUG, BATCH, T, SGS>(a, c, sm, e, live);
+}
+
+template <int K, int M, typename T>
+void fill_face_ops(const DeviceCase &dc, FaceOps<K, M, T> &op)
+{
+  fill_even_odd(dc.opA, op.a);
+  fill_even_odd(dc.opD, op.d);
+  for (int i = 0; i < M * K; ++i) { op.A[i] = T(dc.opA[i]); op.D[i] = T(dc.opD[i]); }
+  for (int q = 0; q < K; ++q)
+    for (int t = 0; t < 4; ++t) op.F[t][q] = T(dc.opF[t][q]);
+  for (int q = 0; q < M; ++q) op.w[q] = dc.opW[q];
+  op.c03 = dc.opC0[0] * dc.opC0[0] * dc.opC0[0];
+}
+
+template <int K, int M, bool BATCH, typename T, bool SGS>
+void launch_face_kernel(bool bug, int n, FaceArgs<K, M, T> &a, hipStream_t s)
+{
+  constexpr int NF = FaceSmem<K, M, T>::NF;
+  a.n = n;
+  if (bug)
+    hipLaunchKernelGGL((face_kernel<K, M, true, BATCH, T, SGS>), dim3((n + NF - 1) / NF, 3), dim3(64), 0, s, a);
+  else
+    hipLaunchKernelGGL((face_kernel<K, M, false, BATCH, T, SGS>), dim3((n + NF - 1) / NF, 3), dim3(64), 0, s, a);
+}
+
+template <int K, int M, typename T>
+hipError_t faces_impl_t(const DeviceCase &dc, hipStream_t s)
+{
+  FaceArgs<K, M, T> a{};
+  a.c = case_dev(dc);
+  fill_face_ops(dc, a.op);
+  if (dc.sgs) launch_face_kernel<K, M, false, T, true>(dc.bug_compat, dc.nElem, a, s);
+  else launch_face_kernel<K, M, false, T, false>(dc.bug_compat, dc.nElem, a, s);
+  return hipGetLastError();
+}
+
+template <int K, int M, typename T>
+hipError_t batch_faces_impl_t(const BatchGroup &g, int w0, int nw, hipStream_t s)
+{
+  FaceArgs<K, M, T> a{};
+  a.cases = g.cases; a.work = g.work; a.w0 = w0;
+  fill_face_ops(*g.proto, a.op);
+  if (g.proto->sgs) launch_face_kernel<K, M, true, T, true>(g.proto->bug_compat, nw, a, s);
+  else launch_face_kernel<K, M, true, T, false>(g.proto->bug_compat, nw, a, s);
+  return hipGetLastError();
+}
+
+}  // namespace
+
+template <int K, int M>
+hipError_t faces(const DeviceCase &dc, hipStream_t s)
+{
+  return dc.mixed ? faces_impl_t<K, M, float>(dc, s) : faces_impl_t<K, M, double>(dc, s);
+}
+
+template <int K, int M>
+hipError_t batch_faces(const BatchGroup &g, int w0, int nw, hipStream_t s)
+{
+  return g.proto->mixed ? batch_faces_impl_t<K, M, float>(g, w0, nw, s)
+                        : batch_faces_impl_t<K, M, double>(g, w0, nw, s);
+}
+
+template hipError_t faces<VCP_SHAPE_K, VCP_SHAPE_M>(const DeviceCase &, hipStream_t);
+template hipError_t batch_faces<VCP_SHAPE_K, VCP_SHAPE_M>(const BatchGroup &, int, int, hipStream_t);
+
+}  // namespace vcp

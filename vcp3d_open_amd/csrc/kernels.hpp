@@ -159,6 +159,16 @@ struct BatchGroup {
   int nt = 0;                       // volume workgroup size, 0: the default
 };
 
+// Volume workgroup sizes instantiated per (K, M): first the column kernel,
+// named by the threads of a plane of points (volume.hip), then the sizes of
+// volume_kernel for which the points fit two passes and the modes one thread
+// each, the fastest first.
+#define VCP_COL_TILES(X) X(3, 4, 16) X(4, 5, 32) X(4, 6, 64) X(5, 7, 64) X(6, 8, 64) X(7, 9, 128)
+#define VCP_TILES(X)                                                            \
+  X(3, 4, 64) X(3, 4, 128) X(3, 4, 256) X(4, 5, 128) X(4, 5, 256)              \
+  X(4, 6, 256) X(4, 6, 128) X(5, 7, 256) X(5, 7, 512) X(6, 8, 256) X(6, 8, 512) \
+  X(7, 9, 512)
+
 bool supported_pair(int K, int M);
 // Volume workgroup sizes available for (K, M); the first is the default.
 int volume_tiles(int K, int M, int out[4]);
@@ -168,8 +178,17 @@ hipError_t launch_faces(const DeviceCase &dc, hipStream_t s);
 // with monitor, also the wall forces into scal[kScalForce ..]
 hipError_t launch_boundary(const DeviceCase &dc, hipStream_t s, bool monitor = false);
 hipError_t launch_volume(const DeviceCase &dc, const StageCtl &ctl, hipStream_t s);
-// the volume kernel with one thread per column of points (volume.hip), one
-// instantiation per supported pair
+// per supported pair: the faces (face.hip), the volume kernel with one
+// workgroup per element (volume_workgroup.hip; nt: its size) and the one with
+// one thread per column of points (volume.hip)
+template <int K, int M>
+hipError_t faces(const DeviceCase &dc, hipStream_t s);
+template <int K, int M>
+hipError_t batch_faces(const BatchGroup &g, int w0, int nw, hipStream_t s);
+template <int K, int M>
+hipError_t volume_workgroup(const DeviceCase &dc, int nt, const StageCtl &ctl, hipStream_t s);
+template <int K, int M>
+hipError_t batch_volume_workgroup(const BatchGroup &g, int nt, const StageCtl &ctl, int w0, int nw, hipStream_t s);
 template <int K, int M>
 hipError_t volume_cols(const DeviceCase &dc, bool full, const StageCtl &ctl, hipStream_t s);
 template <int K, int M>

@@ -9,6 +9,7 @@
 //   SolverClass::ExecuteTimeSynchronizationStep  SolverClass.cpp:2385-2393
 #include "device.hpp"
 #include "kernels.hpp"
+#include "transforms.hpp"
 
 #include <cstdint>
 #include <type_traits>
@@ -16,40 +17,6 @@
 namespace vcp {
 namespace {
 
-// Pointer into constant memory: wave-uniform reads through it are scalar loads.
-template <class X>
-using cptr = const X __attribute__((address_space(4))) *;
-// Pointer into global memory (not flat: a flat access would be counted with
-// the LDS operations in flight).
-template <class X>
-using gptr = X __attribute__((address_space(1))) *;
-template <class X>
-__device__ __forceinline__ gptr<X> glob(X *p) { return (gptr<X>) (uintptr_t) p; }
-
-// ------------------------------------------------- even-odd 1D transforms
-// The operator A in even-odd form, held in scalar registers over the loops
-// that use it (18 doubles at (5, 7)): even modes at the points of the first
-// half and the middle, odd modes at the points of the first half.
-template <int K, int M, typename T>
-struct EvenOdd {
-  static constexpr int HE = (M + 1) / 2, HO = M / 2, KE = (K + 1) / 2, KO = K / 2;
-  T e[HE * KE], o[HO * KO];
-};
-
-template <int K, int M, typename T>
-__device__ __forceinline__ EvenOdd<K, M, T> scalar_op(cptr<EvenOdd<K, M, T>> p)
-{
-  EvenOdd<K, M, T> a;
-#pragma unroll
-  for (int i = 0; i < a.HE * a.KE; ++i) { a.e[i] = p->e[i]; asm volatile("" : "+s"(a.e[i])); }
-#pragma unroll
-  for (int i = 0; i < a.HO * a.KO; ++i) { a.o[i] = p->o[i]; asm volatile("" : "+s"(a.o[i])); }
-  return a;
-}
-
-// The 1D operators as kernel arguments. The Gauss points are symmetric about
-// 0 and phi_q has the parity of q, so A and D need only their first (M+1)/2
-// rows wherever a whole line is transformed (even-odd form).
 // Derivative of the Lagrange polynomials of the Gauss points, C[a][b] =
 // l_b'(r_a), centro-antisymmetric: P and Q hold (C[a][b] +- C[a][M-1-b]) / 2
 // for a, b < M/2, cm its middle column and mr its middle row (odd M).
@@ -59,6 +26,7 @@ struct LineDeriv {
   double P[H * H], Q[H * H], cm[H], mr[H];
 };
 
+// The 1D operators as kernel arguments.
 template <int K, int M, typename T>
 struct ColOps {
   EvenOdd<K, M, T> a;
@@ -82,53 +50,6 @@ struct ColArgs {
   int oW2, oCentre, oFace;     // offsets in the table block: w2, basis at the element centre, face vectors
   ColOps<K, M, T> op;
 };
-
-// modes -> points: o[p] = sum_q A[p][q] c[q]
-template <int K, int M, typename T>
-__device__ __forceinline__ void to_points(const EvenOdd<K, M, T> &A, const T (&c)[K], T (&o)[M])
-{
-  using E = EvenOdd<K, M, T>;
-#pragma unroll
-  for (int p = 0; p < E::HE; ++p) {
-    T e = A.e[p * E::KE] * c[0];
-#pragma unroll
-    for (int q = 1; q < E::KE; ++q) e += A.e[p * E::KE + q] * c[2 * q];
-    if (p < E::HO) {
-      T d = A.o[p * E::KO] * c[1];
-#pragma unroll
-      for (int q = 1; q < E::KO; ++q) d += A.o[p * E::KO + q] * c[2 * q + 1];
-      o[p] = e + d;
-      o[M - 1 - p] = e - d;
-    } else {
-      o[p] = e;
-    }
-  }
-}
-
-// points -> modes: o[q] = sum_p A[p][q] x[p]
-template <int K, int M, typename T>
-__device__ __forceinline__ void to_modes(const EvenOdd<K, M, T> &A, const T (&x)[M], T (&o)[K])
-{
-  using E = EvenOdd<K, M, T>;
-  T s[E::HE], d[E::HO];
-#pragma unroll
-  for (int p = 0; p < E::HO; ++p) { s[p] = x[p] + x[M - 1 - p]; d[p] = x[p] - x[M - 1 - p]; }
-  if constexpr (M % 2) s[E::HO] = x[E::HO];
-#pragma unroll
-  for (int q = 0; q < E::KE; ++q) {
-    T v = A.e[q] * s[0];
-#pragma unroll
-    for (int p = 1; p < E::HE; ++p) v += A.e[p * E::KE + q] * s[p];
-    o[2 * q] = v;
-  }
-#pragma unroll
-  for (int q = 0; q < E::KO; ++q) {
-    T v = A.o[q] * d[0];
-#pragma unroll
-    for (int p = 1; p < E::HO; ++p) v += A.o[p * E::KO + q] * d[p];
-    o[2 * q + 1] = v;
-  }
-}
 
 // derivative along a line of M point values, in place; TRANS: its transpose.
 // In double in both forms: the nodal derivative cancels the constant part of
@@ -169,40 +90,6 @@ __device__ __forceinline__ void line_deriv(cptr<LineDeriv<M>> op, double (&x)[M]
 // or two waves. Sum (the first NS values) or max of non-negative values; the
 // result is returned to every thread. Two-wave groups exchange their partial
 // results through alternating halves of red, with one barrier.
-template <int CTRL>
-__device__ __forceinline__ double dpp_all_f64(double v)
-{
-  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), CTRL, 0xf, 0xf, true);
-  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), CTRL, 0xf, 0xf, true);
-  return __hiloint2double(hi, lo);
-}
-
-template <int G, bool MAX>
-__device__ __forceinline__ double lanes_reduce(double v)
-{
-  if constexpr (G >= 64) return wave_reduce_dpp<MAX>(v);
-  auto op = [](double x, double y) { return MAX ? fmax(x, y) : x + y; };
-  v = op(v, dpp_all_f64<0xB1>(v));     // quad_perm 1,0,3,2
-  v = op(v, dpp_all_f64<0x4E>(v));     // quad_perm 2,3,0,1
-  v = op(v, dpp_all_f64<0x141>(v));    // row_half_mirror
-  v = op(v, dpp_all_f64<0x140>(v));    // row_mirror
-  if constexpr (G == 32) v = op(v, __shfl_xor(v, 16, 64));
-  return v;
-}
-
-template <int G>
-__device__ __forceinline__ void group_sync()
-{
-  if constexpr (G > 64) {
-    __syncthreads();
-  } else {
-    // one wave: its LDS operations complete in order, so only the compiler
-    // has to keep them in program order
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-  }
-}
-
 template <int G, int NV, int NS>
 __device__ __forceinline__ void group_reduce(double (&v)[NV], double *red, int &half)
 {
@@ -685,9 +572,8 @@ void volume_cols_kernel(ColArgs<K, M, T> args_)
 #pragma unroll
       for (int v = 0; v < 5; ++v) Vp[v] = double(V[v]) + meanPt[v];
       const double *gx = g[0], *gy = g[1], *gz = g[2];
-      double rho, u, v, w, p, eKin;
-      ent2prim(Vp, rho, u, v, w, p, eKin);
-      const double V4Inv = 1.0 / Vp[4];
+      const EntState st = ent_state(Vp);
+      const double rho = st.rho, u = st.u, v = st.v, w = st.w, p = st.p, eKin = st.ek, V4Inv = -st.r;
       const double rE = p * kInvGm1 + rho * eKin;
       const double dudx = -V4Inv * (gx[1] + u * gx[4]), dudy = -V4Inv * (gy[1] + u * gy[4]), dudz = -V4Inv * (gz[1] + u * gz[4]);
       const double dvdx = -V4Inv * (gx[2] + v * gx[4]), dvdy = -V4Inv * (gy[2] + v * gy[4]), dvdz = -V4Inv * (gz[2] + v * gz[4]);
@@ -819,16 +705,14 @@ void volume_cols_kernel(ColArgs<K, M, T> args_)
     }
 #pragma unroll
     for (int p = 0; p < HP; ++p) {
-      const double V4 = double(V[4][p]) + meanPt[4], V4Inv = 1.0 / V4;
-      const double u = -V4Inv * (double(V[1][p]) + meanPt[1]), v = -V4Inv * (double(V[2][p]) + meanPt[2]),
-                   w = -V4Inv * (double(V[3][p]) + meanPt[3]);
-      const double eKin = 0.5 * (u * u + v * v + w * w);
-      const double s = kGam - kGm1 * (double(V[0][p]) + meanPt[0] - V4 * eKin);
-      const double rho = pow_m2p5(-V4 * exp(s));
+      double Vp[5];
+#pragma unroll
+      for (int l = 0; l < 5; ++l) Vp[l] = double(V[l][p]) + meanPt[l];
+      const EntState st = ent_state(Vp);
       // the middle plane of an odd M belongs to the first half
       const bool mine = H == 1 || M % 2 == 0 || p < HP - 1 || h == 0;
-      pr[p][0] = mine ? T(w2 * op->w[p] * J[p] * rho) : T(0);
-      pr[p][1] = T(u); pr[p][2] = T(v); pr[p][3] = T(w); pr[p][4] = T(-V4Inv);
+      pr[p][0] = mine ? T(w2 * op->w[p] * J[p] * st.rho) : T(0);
+      pr[p][1] = T(st.u); pr[p][2] = T(st.v); pr[p][3] = T(st.w); pr[p][4] = T(st.r);
 #pragma unroll
       for (int l = 0; l < 5; ++l) asm volatile("" : "+v"(pr[p][l]));
       __builtin_amdgcn_sched_barrier(0);
@@ -1084,17 +968,8 @@ void fill_col_args(const DeviceCase &dc, const StageCtl &ctl, ColArgs<K, M, T> &
     a.op.A[i] = T(dc.opA[i]); a.op.D[i] = T(dc.opD[i]);
     a.op.Ad[i] = dc.opA[i]; a.op.Dd[i] = dc.opD[i];
   }
-  using E = EvenOdd<K, M, T>;
-  for (int p = 0; p < E::HE; ++p)
-    for (int q = 0; q < K; ++q) {
-      if (q % 2 == 0) {
-        a.op.a.e[p * E::KE + q / 2] = T(dc.opA[p * K + q]);
-        a.op.ad.e[p * E::KE + q / 2] = dc.opA[p * K + q];
-      } else if (p < E::HO) {
-        a.op.a.o[p * E::KO + q / 2] = T(dc.opA[p * K + q]);
-        a.op.ad.o[p * E::KO + q / 2] = dc.opA[p * K + q];
-      }
-    }
+  fill_even_odd(dc.opA, a.op.a);
+  fill_even_odd(dc.opA, a.op.ad);
   for (int p = 0; p < H; ++p) {
     for (int q = 0; q < H; ++q) {
       const double l = dc.opDL[p * M + q], m = dc.opDL[p * M + M - 1 - q];
