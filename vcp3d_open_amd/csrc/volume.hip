@@ -323,7 +323,8 @@ void volume_cols_kernel(ColArgs<K, M, T> args_)
   T *const XS = lds + S::S + t;                 // kTight: x of mode slot s, variable l at (s * 5 + l) * G
   const auto Ue = glob((const double *) a->U) + (size_t) e * 5 * ND;
   const auto vg = glob(a->vgeo) + (size_t) e * kVolGeo * NI;
-  const int sp = FULL && a->spIdx ? glob(a->spIdx)[e] : -1;
+  int sp = FULL && a->spIdx ? glob(a->spIdx)[e] : -1;
+  if constexpr (kUniform) sp = __builtin_amdgcn_readfirstlane(sp);
   const bool act = tl < N2;
   const int col = act ? tl : 0, ci = col % M, cj = col / M, colT = ci * M + cj;
   const T sgn = T(h ? -1 : 1);
@@ -485,6 +486,121 @@ void volume_cols_kernel(ColArgs<K, M, T> args_)
   const bool cml = FULL && sp >= 0 && a->cml;
   double mach2 = 0.0, evMax = 0.0;
   const int np = H == 1 ? M : h ? M / 2 : (M + 1) / 2;
+  // entropy variables and their derivatives along k at this thread's point of
+  // plane k
+  auto plane_values = [&](int k, T (&V)[5], T (&Gt)[5]) {
+    const auto op = ops();
+    cptr<T> Ak = op->A + k * K, Dk = op->D + k * K;
+#pragma unroll
+    for (int v = 0; v < 5; ++v) {
+      T c[K];
+#pragma unroll
+      for (int q = 0; q < K; ++q) c[q] = X[(v * K + q) * NP + col];
+      T s = Ak[0] * c[0], d = Dk[1] * c[1];
+#pragma unroll
+      for (int q = 1; q < K; ++q) { s += Ak[q] * c[q]; if (q > 1) d += Dk[q] * c[q]; }
+      V[v] = s; Gt[v] = d;
+    }
+  };
+  // derivative (transposed: TRANS) of lines [0, NL) of the half, in place
+  auto derive_lines = [&](auto nl, auto trans) {
+    constexpr int NL = decltype(nl)::value;
+    const auto ld = &ops()->l;
+#pragma unroll
+    for (int r = 0; r < (NL + LH - 1) / LH; ++r) {
+      const int l = tl + r * LH;
+      if (l < NL) {
+        double *x = PB + (l / M) * NP + (l % M) * M;
+        double y[M];
+#pragma unroll
+        for (int p = 0; p < M; ++p) y[p] = x[p];
+        line_deriv<M, decltype(trans)::value>(ld, y);
+#pragma unroll
+        for (int p = 0; p < M; ++p) x[p] = y[p];
+      }
+    }
+  };
+  // Cartesian gradient of variable v from its parametric derivatives
+  auto cartesian = [&](int v, double gr, double gs, double gt, const double (&cur)[kVolGeo], double (&g)[3][5]) {
+    cptr<double> vs = (cptr<double>) (uintptr_t) (vg + NI);
+#pragma unroll
+    for (int x = 0; x < 3; ++x) {
+      if (!args->bug)
+        g[x][v] = gr * cur[1 + x] + gs * cur[4 + x] + gt * cur[7 + x];
+      else if constexpr (kUniform)
+        g[x][v] = gr * vs[x * NI + v] + gs * vs[(3 + x) * NI + v] + gt * vs[(6 + x) * NI + v];
+      else
+        g[x][v] = gr * sCm[sub][v * 9 + x] + gs * sCm[sub][v * 9 + 3 + x] + gt * sCm[sub][v * 9 + 6 + x];
+    }
+  };
+  // ---------------- sponge, matching-layer and body-force sources, in planes
+  // of their own ahead of the fluxes': beside the fluxes they spill 40
+  // registers in every element, of those outside the sponge too. Volume launch
+  // of the 48 x 24 x 24 open box at (5, 7), 8 of 48 element layers in the
+  // sponge: 888 us beside the fluxes, 718 us here; 18^3 (3, 4) with WALE,
+  // which these sources spilled as well: 57 / 53 us.
+  if constexpr (FULL)
+    if (sp >= 0 || a->bfBuf) {
+#pragma unroll 1
+      for (int pl = 0; pl < (LH > 64 ? HP : np); ++pl) {
+        const bool valid = LH <= 64 || pl < np;
+        const int k = H == 2 && h ? M - 1 - pl : pl, m = k * N2 + col;
+        double cur[kVolGeo];
+#pragma unroll
+        for (int q = 0; q < kVolGeo; ++q) cur[q] = vg[(unsigned) (q * NI + m)];
+        T V[5], Gt[5];
+        plane_values(k, V, Gt);
+        double g[3][5];
+        if (cml) {
+          if (act)
+#pragma unroll
+            for (int v = 0; v < 5; ++v) { PB[v * NP + tl] = V[v]; PB[(5 + v) * NP + colT] = V[v]; }
+          group_sync<LH>();
+          derive_lines(std::integral_constant<int, 10 * M>{}, std::false_type{});
+          group_sync<LH>();
+#pragma unroll
+          for (int v = 0; v < 5; ++v) cartesian(v, PB[v * NP + col], PB[(5 + v) * NP + colT], Gt[v], cur, g);
+        }
+        double Vp[5];
+#pragma unroll
+        for (int v = 0; v < 5; ++v) Vp[v] = double(V[v]) + meanPt[v];
+        const EntState st = ent_state(Vp);
+        const double wJ = w2 * args->op.w[k] * cur[0], weight = -wJ;
+        double src[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+        if (sp >= 0) {
+          // sponge damping sigma J w (U - U_target) and CML sources
+          // (ElementClass.cpp:4450-4489, :3887-4117)
+          const auto fn = glob(a->dampFn) + (size_t) sp * 3 * NI, ds = glob(a->dampState) + (size_t) sp * 5 * NI;
+          const double sigma = wJ * (fn[m] + fn[NI + m] + fn[2 * NI + m]);
+          src[0] = sigma * (st.rho - ds[m]);
+          src[1] = sigma * (st.rho * st.u - ds[NI + m]);
+          src[2] = sigma * (st.rho * st.v - ds[2 * NI + m]);
+          src[3] = sigma * (st.rho * st.w - ds[3 * NI + m]);
+          src[4] = sigma * (st.p * kInvGm1 + st.rho * st.ek - ds[4 * NI + m]);
+          if (cml) {
+            const auto cf = glob(a->spCoef) + (size_t) sp * 8;
+            const double wgt[3] = {weight * cf[0] * fn[m], weight * cf[1] * fn[NI + m], weight * cf[2] * fn[2 * NI + m]};
+            const double nsg[3] = {cf[3], cf[4], cf[5]};
+            cml_source(Vp, g[0], g[1], g[2], wgt, nsg, src);
+          }
+        }
+        if (a->bfBuf) {
+          // body force per unit volume (ElementClass.cpp:4492-4523): -w J f on
+          // the momentum and -w J u.f on the energy equation
+          const double bx = a->fbody[0], by = a->fbody[1], bz = a->fbody[2];
+          src[1] += weight * bx; src[2] += weight * by; src[3] += weight * bz;
+          src[4] += weight * (st.u * bx + st.v * by + st.w * bz);
+        }
+        if (valid) {
+          cptr<double> Ak = ops()->Ad + k * K;
+#pragma unroll
+          for (int v = 0; v < 5; ++v)
+#pragma unroll
+            for (int q = 0; q < K; ++q) acc[v][q] += Ak[q] * src[v];
+        }
+        group_sync<LH>();
+      }
+    }
 #pragma unroll 1
   for (int pl = 0; pl < (LH > 64 ? HP : np); ++pl) {
     const bool valid = LH <= 64 || pl < np;      // equal trips where the halves share barriers
@@ -493,79 +609,18 @@ void volume_cols_kernel(ColArgs<K, M, T> args_)
 #pragma unroll
     for (int q = 0; q < kVolGeo; ++q) cur[q] = vg[(unsigned) (q * NI + k * N2 + col)];
     T V[5], Gt[5];
-    {
-      const auto op = ops();
-      cptr<T> Ak = op->A + k * K, Dk = op->D + k * K;
-#pragma unroll
-      for (int v = 0; v < 5; ++v) {
-        T c[K];
-#pragma unroll
-        for (int q = 0; q < K; ++q) c[q] = X[(v * K + q) * NP + col];
-        T s = Ak[0] * c[0], d = Dk[1] * c[1];
-#pragma unroll
-        for (int q = 1; q < K; ++q) { s += Ak[q] * c[q]; if (q > 1) d += Dk[q] * c[q]; }
-        V[v] = s; Gt[v] = d;
-      }
-    }
+    plane_values(k, V, Gt);
     // lines along i (slots 0..3) and along j (4..7) of variables 1..4
     if (act)
 #pragma unroll
       for (int v = 0; v < 4; ++v) { PB[v * NP + tl] = V[1 + v]; PB[(4 + v) * NP + colT] = V[1 + v]; }
-    if (FULL && cml && act) { PB[8 * NP + tl] = V[0]; PB[9 * NP + colT] = V[0]; }
     group_sync<LH>();
-    {
-      const auto ld = &ops()->l;
-#pragma unroll
-      for (int r = 0; r < (8 * M + LH - 1) / LH; ++r) {
-        const int l = tl + r * LH;
-        if (l < 8 * M) {
-          double *x = PB + (l / M) * NP + (l % M) * M;
-          double y[M];
-#pragma unroll
-          for (int p = 0; p < M; ++p) y[p] = x[p];
-          line_deriv<M, false>(ld, y);
-#pragma unroll
-          for (int p = 0; p < M; ++p) x[p] = y[p];
-        }
-      }
-      if (FULL && cml && tl < 2 * M) {
-        double *x = PB + (8 + tl / M) * NP + (tl % M) * M;
-        double y[M];
-#pragma unroll
-        for (int p = 0; p < M; ++p) y[p] = x[p];
-        line_deriv<M, false>(ld, y);
-#pragma unroll
-        for (int p = 0; p < M; ++p) x[p] = y[p];
-      }
-    }
+    derive_lines(std::integral_constant<int, 8 * M>{}, std::false_type{});
     group_sync<LH>();
     double g[3][5];                                   // Cartesian gradients
-    g[0][0] = g[1][0] = g[2][0] = 0.0;
-    {
-      cptr<double> vs = (cptr<double>) (uintptr_t) (vg + NI);
 #pragma unroll
-      for (int v = 0; v < 5; ++v) {
-        if (v == 0 && !(FULL && cml)) continue;
-        const int slot = v == 0 ? 8 : v - 1, slotT = v == 0 ? 9 : v + 3;
-        const double gr = PB[slot * NP + col], gs = PB[slotT * NP + colT], gt = Gt[v];
-        if (args->bug) {
-#pragma unroll
-          for (int x = 0; x < 3; ++x) {
-            {
-              if constexpr (kUniform)
-                g[x][v] = gr * vs[x * NI + v] + gs * vs[(3 + x) * NI + v] + gt * vs[(6 + x) * NI + v];
-              else
-                g[x][v] = gr * sCm[sub][v * 9 + x] + gs * sCm[sub][v * 9 + 3 + x] + gt * sCm[sub][v * 9 + 6 + x];
-            }
-          }
-        } else {
-#pragma unroll
-          for (int x = 0; x < 3; ++x) g[x][v] = gr * cur[1 + x] + gs * cur[4 + x] + gt * cur[7 + x];
-        }
-      }
-    }
+    for (int v = 1; v < 5; ++v) cartesian(v, PB[(v - 1) * NP + col], PB[(v + 3) * NP + colT], Gt[v], cur, g);
     double Ft[5];
-    double src[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
     {
       double Fr[5], Fs[5];
       double Vp[5];
@@ -612,36 +667,6 @@ void volume_cols_kernel(ColArgs<K, M, T> args_)
           else Ft[l] = F;
         }
       }
-      if constexpr (FULL) {
-        double so[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-        if (sp >= 0) {
-          // sponge damping sigma J w (U - U_target) and CML sources
-          // (ElementClass.cpp:4450-4489, :3887-4117)
-          const int m = k * N2 + col;
-          const auto fn = glob(a->dampFn) + (size_t) sp * 3 * NI, ds = glob(a->dampState) + (size_t) sp * 5 * NI;
-          const double sigma = wJ * (fn[m] + fn[NI + m] + fn[2 * NI + m]);
-          so[0] = sigma * (rho - ds[m]);
-          so[1] = sigma * (ru - ds[NI + m]);
-          so[2] = sigma * (rv - ds[2 * NI + m]);
-          so[3] = sigma * (rw - ds[3 * NI + m]);
-          so[4] = sigma * (rE - ds[4 * NI + m]);
-          if (cml) {
-            const auto cf = glob(a->spCoef) + (size_t) sp * 8;
-            const double wgt[3] = {weight * cf[0] * fn[m], weight * cf[1] * fn[NI + m], weight * cf[2] * fn[2 * NI + m]};
-            const double nsg[3] = {cf[3], cf[4], cf[5]};
-            cml_source(Vp, gx, gy, gz, wgt, nsg, so);
-          }
-        }
-        if (a->bfBuf) {
-          // body force per unit volume (ElementClass.cpp:4492-4523): -w J f on
-          // the momentum and -w J u.f on the energy equation
-          const double bx = a->fbody[0], by = a->fbody[1], bz = a->fbody[2];
-          so[1] += weight * bx; so[2] += weight * by; so[3] += weight * bz;
-          so[4] += weight * (u * bx + v * by + w * bz);
-        }
-#pragma unroll
-        for (int l = 0; l < 5; ++l) src[l] = so[l];
-      }
       // in-plane fluxes: lines along i of the r fluxes (slots 0..4) and along j
       // of the s fluxes (5..9), contracted with the transposed derivative; they
       // overwrite the gradients once every thread has read its own
@@ -651,30 +676,14 @@ void volume_cols_kernel(ColArgs<K, M, T> args_)
         for (int l = 0; l < 5; ++l) { PB[l * NP + tl] = Fr[l]; PB[(5 + l) * NP + colT] = Fs[l]; }
     }
     group_sync<LH>();
-    {
-      const auto ld = &ops()->l;
-#pragma unroll
-      for (int r = 0; r < (10 * M + LH - 1) / LH; ++r) {
-        const int l = tl + r * LH;
-        if (l < 10 * M) {
-          double *x = PB + (l / M) * NP + (l % M) * M;
-          double y[M];
-#pragma unroll
-          for (int p = 0; p < M; ++p) y[p] = x[p];
-          line_deriv<M, true>(ld, y);
-#pragma unroll
-          for (int p = 0; p < M; ++p) x[p] = y[p];
-        }
-      }
-    }
+    derive_lines(std::integral_constant<int, 10 * M>{}, std::true_type{});
     group_sync<LH>();
     if (valid) {
       const auto op = ops();
       cptr<double> Ak = op->Ad + k * K, Dk = op->Dd + k * K;
 #pragma unroll
       for (int v = 0; v < 5; ++v) {
-        double s = PB[v * NP + col] + PB[(5 + v) * NP + colT];
-        if constexpr (FULL) s += src[v];
+        const double s = PB[v * NP + col] + PB[(5 + v) * NP + colT];
 #pragma unroll
         for (int q = 0; q < K; ++q) {
           acc[v][q] += Ak[q] * s;
