@@ -37,16 +37,14 @@ struct FaceArgs {
 
 // ============================================================ face kernel
 // Faces in direction DIR: each lane group of a wave (the wave, or 32 or 16
-// lanes where the M^2 points fill only that many) takes one element's min
-// face. Side 0 is the element itself (its min face), side 1 the neighbour L
-// (its max face); the normal points from L to the element. When the fast
-// contraction (2 * 5 K columns) and the points (M^2) fit the wave, those
-// phases overwrite their own input in place (every line is read before any is
-// stored); otherwise (K = 7, M = 9) T gets a region of its own. LDS regions:
+// lanes where the M^2 points fill only that many; two waves at M = 9) takes
+// one element's min face. Side 0 is the element itself (its min face), side 1 the neighbour L
+// (its max face); the normal points from L to the element. Every phase reads
+// all of its lines before it stores over them. LDS regions:
 //   X: normal contraction B -> fast contraction T -> flux and Cartesian
-//      symmetrising fluxes at the points (over B, or over T when in place)
-//   Y: the first lift stage of one side: flux + fast slot of five variables,
-//      slow slot and normal slot of variables 1..4
+//      symmetrising fluxes at the points
+//   Y: behind the fluxes in X, the first lift stage of one side: flux + fast
+//      slot of five variables, slow slot and normal slot of variables 1..4
 //
 // What bounds it: instruction issue and latency at three waves per SIMD (LDS),
 // not memory. The line contractions use the even-odd operators, the lift
@@ -57,36 +55,41 @@ struct FaceArgs {
 // of a Taylor-Green case before / after, us: (3, 4) 18^3 72 / 43,
 // (4, 5) 16^3 68 / 48, (4, 6) 14^3 54 / 46, (5, 7) 32^3 612 / 530,
 // (6, 8) 16^3 194 / 133, (7, 9) 14^3 232 / 214; mixed (3, 4) 71 / 34,
-// (5, 7) 498 / 437.
+// (5, 7) 498 / 437. With the odd pitches and two waves per face at M = 9 below,
+// then: (6, 8) 16^3 130 / 106, (7, 9) 11^3 98 / 68, the others within 3 %.
 template <int K, int M, typename T = double>
 struct FaceSmem {
   // faces per wave and lanes per face: the pointwise fluxes are half of the
   // instructions, and the M^2 points of one face leave most of a wave idle at
   // M = 4 and 5 ((3, 4) 18^3: 57 us with one face per wave, 43 with four)
-  static constexpr int NF = M * M <= 16 ? 4 : M * M <= 32 ? 2 : 1, G = 64 / NF;
-  static constexpr bool kInPlace = 2 * 5 * K <= 64 && M * M <= 64;
+  static constexpr int NF = M * M <= 16 ? 4 : M * M <= 32 ? 2 : 1;
+  // threads of the workgroup, and per face: the 81 points of M = 9 take two
+  // waves. (In one wave they take two passes, the second with 17 lanes, and the
+  // fast contraction's output a region of its own, which leaves four waves per
+  // CU: launch over 3457 elements 240 us, in two waves 155.)
+  static constexpr int NT = M * M > 64 ? 128 : 64, G = NT / NF;
+  static_assert(M * M <= G, "the points of a face in one pass");
   // traces: the value of five variables, the fast and normal derivatives of
   // variables 1..4 (the fluxes need no gradient of the first); points: the
-  // flux of five variables, the symmetrising fluxes of 1..4 (the first's are 0)
-  static constexpr int kB = 2 * 2 * 5 * K * K, kT1 = 13 * K * M, kT = 2 * kT1, kP = 17 * M * M;
-  static constexpr int kOffT = kInPlace ? 0 : cmax(kB, kP);   // the fluxes start at 0
-  static constexpr int kX = kInPlace ? cmax(cmax(kB, kT), kP) : kOffT + kT;
-  static constexpr int kY = 13 * M * K;
-  static constexpr int kBytes = (int) sizeof(T) * (2 * M * K + 4 * K + NF * (kX + kY)) + 8 * (M * M + NF * 82);
-  // waves per SIMD to compile for: three when 12 faces fit a CU's 160 KB
-#ifndef VCP_F32_FACE_WAVES
-#define VCP_F32_FACE_WAVES 3
-#endif
-  static constexpr int kWaves = sizeof(T) == 4 && 4 * VCP_F32_FACE_WAVES * kBytes <= 160 * 1024 ? VCP_F32_FACE_WAVES
-                                : 12 * kBytes <= 160 * 1024 ? 3 : 2;
+  // flux of five variables, the symmetrising fluxes of 1..4 (the first's are
+  // 0). Lines of K and M values at odd pitches: lanes that take neighbouring
+  // lines fall into different banks (at (6, 8) more than half of the LDS cycles
+  // were conflicts, and the LDS 80 % busy)
+  static constexpr int KP = K | 1, MP = M | 1, NP = M * MP;
+  static constexpr int kB = 2 * 2 * 5 * K * KP, kT1 = 13 * K * MP, kT = 2 * kT1, kP = 17 * NP;
+  static constexpr int kY = 13 * M * KP;
+  static constexpr int kX = cmax(cmax(kB, kT), kP + kY);
+  static constexpr int kBytes = (int) sizeof(T) * (2 * M * K + 4 * K + NF * kX) + 8 * (M * M + 1 + NF * 82);
+  // waves per SIMD to compile for: three when 12 waves fit a CU's 160 KB
+  static constexpr int kWaves = 12 * 64 / NT * kBytes <= 160 * 1024 ? 3 : 2;
   T A[M * K], D[M * K];
   double W2[M * M];
   T F[4][K];                       // phi(-1), phi(+1), phi'(-1), phi'(+1)
+  double EvMax;                    // the second wave's eddy-viscosity maximum (two waves per face)
   struct Face {
     double Cm[2][4][9];            // metric of points 1..4 (bug)
     double Mean[2][5];             // float form: mode 0 of both elements
     T X[kX];
-    T Y[kY];
   } f[NF];
 };
 
@@ -111,7 +114,8 @@ __device__ __forceinline__ void face_body(const FaceArgs<K, M, T> &args, const C
   if (L < 0) L = e;
   constexpr int ND = K * K * K, N2 = M * M;
   using S = FaceSmem<K, M, T>;
-  constexpr int G = S::G;
+  constexpr int G = S::G, NT = S::NT, KP = S::KP, MP = S::MP, NP = S::NP;
+  constexpr int SB = 5 * K * KP;              // one plane of B
   // strides of the (normal, fast, slow) axes in the [k][j][i] DOF layout
   constexpr int SN = DIR == 0 ? 1 : DIR == 1 ? K : K * K;
   constexpr int SFA = DIR == 0 ? K : 1;
@@ -120,34 +124,32 @@ __device__ __forceinline__ void face_body(const FaceArgs<K, M, T> &args, const C
   constexpr int PN = DIR, PF = DIR == 0 ? 1 : 0, PS = DIR == 2 ? 1 : 2;
   T *sA = sm.A, *sD = sm.D;
   double *sW2 = sm.W2;
-  const int lane = threadIdx.x, tid = lane % G;   // lane of the wave, of the face
+  const int lane = threadIdx.x, tid = lane % G;   // thread of the workgroup, of the face
   typename S::Face &sf = sm.f[lane / G];
-  T *B = sf.X;                                // [side][value|deriv][5][K][K]
-  T *Tb = sf.X + S::kOffT;                    // [side][A|D|N][5, 4, 4][K][M]
-  T *sFlux = sf.X, *sFC = sf.X + 5 * N2;      // flux [5][N2], Cartesian sym [x|y|z][4][N2] of variables 1..4
+  T *B = sf.X;                                // [side][value|deriv][5][K][KP]
+  T *Tb = sf.X;                               // [side][A|D|N][5, 4, 4][K][MP]
+  T *sFlux = sf.X, *sFC = sf.X + 5 * NP;      // flux [5][M][MP], Cartesian sym [x|y|z][4][M][MP] of variables 1..4
   // operators in LDS: read as wave-uniform LDS operands in the contractions
   // (as kernel arguments they would not fit the scalar registers)
-  for (int i = lane; i < M * K; i += 64) { sA[i] = VCP_FOPS.A[i]; sD[i] = VCP_FOPS.D[i]; }
-  for (int i = lane; i < 4 * K; i += 64) sm.F[i / K][i % K] = VCP_FOPS.F[i / K][i % K];
+  for (int i = lane; i < M * K; i += NT) { sA[i] = VCP_FOPS.A[i]; sD[i] = VCP_FOPS.D[i]; }
+  for (int i = lane; i < 4 * K; i += NT) sm.F[i / K][i % K] = VCP_FOPS.F[i / K][i % K];
   // operators of the line contractions, through scalar loads
   auto ops = [&]() { auto p = (cptr<FaceOps<K, M, T>>) (uintptr_t) &args.op; asm volatile("" : "+s"(p)); return p; };
-  for (int i = lane; i < N2; i += 64) sW2[i] = VCP_FOPS.w[i % M] * VCP_FOPS.w[i / M];
+  for (int i = lane; i < N2; i += NT) sW2[i] = VCP_FOPS.w[i % M] * VCP_FOPS.w[i / M];
   const double *g = a.fgeo + ((size_t) e * 3 + DIR) * kFaceGeo * N2;
   // Loads issued here and used after the contractions, so that their latency
-  // passes under them: the two length scales and, when the points fit the
-  // wave in one pass, this lane's point metric (normal, area and, unless the
-  // metric comes from sm.Cm, both sides' inverse metric).
+  // passes under them: the two length scales and this lane's point
+  // metric (normal, area and, unless the metric comes from sm.Cm, both sides'
+  // inverse metric).
   const double lenE = a.econst[(size_t) e * kElemConst + DIR], lenL = a.econst[(size_t) L * kElemConst + DIR];
-  constexpr bool kGeoEarly = N2 <= G;
+  const bool atPoint = tid < N2;
+  const int m = atPoint ? tid : 0;
   double geoCm[2][9], geoN[4];
-  if constexpr (kGeoEarly) {
-    const int mm = tid < N2 ? tid : 0;
-    if constexpr (!BUG)
+  if constexpr (!BUG)
 #pragma unroll
-      for (int q = 0; q < 9; ++q) { geoCm[0][q] = g[(13 + q) * N2 + mm]; geoCm[1][q] = g[(4 + q) * N2 + mm]; }
+    for (int q = 0; q < 9; ++q) { geoCm[0][q] = g[(13 + q) * N2 + m]; geoCm[1][q] = g[(4 + q) * N2 + m]; }
 #pragma unroll
-    for (int q = 0; q < 4; ++q) geoN[q] = g[q * N2 + mm];
-  }
+  for (int q = 0; q < 4; ++q) geoN[q] = g[q * N2 + m];
   if constexpr (BUG)
 #pragma unroll
     for (int it = 0; it < (72 + G - 1) / G; ++it) {
@@ -159,18 +161,18 @@ __device__ __forceinline__ void face_body(const FaceArgs<K, M, T> &args, const C
     }
   if constexpr (kMixed)
     if (tid < 10) sf.Mean[tid / 5][tid % 5] = a.U[(size_t) (tid < 5 ? e : L) * 5 * ND + (tid % 5) * ND];
-  group_sync<64>();
+  group_sync<NT>();
   // normal contraction straight from HBM: B[side][0|1][v][s][f]; the loads of
   // both sides (K <= 6, at most 40 registers) or of one side at a time (K = 7)
   // are issued before the first of them is waited for. In the float form the
   // mean (mode 0) is added at the points.
   constexpr int NIT = (5 * K * K + G - 1) / G;
-  constexpr int SB = 2 * NIT * K <= 40 ? 2 : 1;
+  constexpr int NS = 2 * NIT * K <= 40 ? 2 : 1;
 #pragma unroll
-  for (int s0 = 0; s0 < 2; s0 += SB) {
-    double xu[SB][NIT][K];
+  for (int s0 = 0; s0 < 2; s0 += NS) {
+    double xu[NS][NIT][K];
 #pragma unroll
-    for (int sb = 0; sb < SB; ++sb) {
+    for (int sb = 0; sb < NS; ++sb) {
       const double *Us = a.U + (size_t) (s0 + sb ? L : e) * 5 * ND;
 #pragma unroll
       for (int it = 0; it < NIT; ++it) {
@@ -182,7 +184,7 @@ __device__ __forceinline__ void face_body(const FaceArgs<K, M, T> &args, const C
       }
     }
 #pragma unroll
-    for (int sb = 0; sb < SB; ++sb) {
+    for (int sb = 0; sb < NS; ++sb) {
       const int side = s0 + sb;
       const T *Fv = sm.F[side], *dFv = sm.F[2 + side];
 #pragma unroll
@@ -196,42 +198,38 @@ __device__ __forceinline__ void face_body(const FaceArgs<K, M, T> &args, const C
             const T x = (kMixed && t == 0 && sl == 0 && f == 0) ? T(0) : T(xu[sb][it][t]);
             b0 += Fv[t] * x; b1 += dFv[t] * x;
           }
-          B[(side * 2 + 0) * 5 * K * K + pc] = b0;
-          B[(side * 2 + 1) * 5 * K * K + pc] = b1;
+          B[(side * 2 + 0) * SB + (pc / K) * KP + f] = b0;
+          B[(side * 2 + 1) * SB + (pc / K) * KP + f] = b1;
         }
       }
     }
   }
-  group_sync<64>();
-  // fast tangential contraction (in place over B when single-pass):
+  group_sync<NT>();
+  // fast tangential contraction, in place over B:
   // T[side][A|D|N][v][s][f'], f' < M
   constexpr int RF = (2 * 5 * K + G - 1) / G;
-  T in[S::kInPlace ? RF : 1][2][K];
-  auto read_line = [&](int r, T (&x)[2][K]) {
+  T in[RF][2][K];
+#pragma unroll
+  for (int r = 0; r < RF; ++r) {
     const int c = tid + r * G;
     if (c < 2 * 5 * K) {
       const int side = c / (5 * K), vs = c - side * 5 * K;
 #pragma unroll
       for (int f = 0; f < K; ++f) {
-        x[0][f] = B[(side * 2 + 0) * 5 * K * K + vs * K + f];
-        x[1][f] = B[(side * 2 + 1) * 5 * K * K + vs * K + f];
+        in[r][0][f] = B[(side * 2 + 0) * SB + vs * KP + f];
+        in[r][1][f] = B[(side * 2 + 1) * SB + vs * KP + f];
       }
     }
-  };
-  if constexpr (S::kInPlace) {
-#pragma unroll
-    for (int r = 0; r < RF; ++r) read_line(r, in[r]);
-    group_sync<64>();
   }
+  group_sync<NT>();
 #pragma unroll
   for (int r = 0; r < RF; ++r) {
-    T (&x)[2][K] = in[S::kInPlace ? r : 0];
-    if constexpr (!S::kInPlace) read_line(r, x);
+    T (&x)[2][K] = in[r];
     const int c = tid + r * G;
     if (c >= 2 * 5 * K) continue;
     const int side = c / (5 * K), vs = c - side * 5 * K;
     // [A: 5 variables][D: 4][N: 4][s][f'], D and N of variables 1..4
-    T *Ts = Tb + side * S::kT1 + vs * M;
+    T *Ts = Tb + side * S::kT1 + vs * MP;
     const auto op = ops();
     const EvenOdd<K, M, T> A = scalar_op<K, M, T>(&op->a);
     T tA[M], tD[M], tN[M];
@@ -242,12 +240,12 @@ __device__ __forceinline__ void face_body(const FaceArgs<K, M, T> &args, const C
     for (int n = 0; n < M; ++n) Ts[n] = tA[n];
     if (vs >= K)
 #pragma unroll
-      for (int n = 0; n < M; ++n) { Ts[4 * K * M + n] = tD[n]; Ts[8 * K * M + n] = tN[n]; }
+      for (int n = 0; n < M; ++n) { Ts[4 * K * MP + n] = tD[n]; Ts[8 * K * MP + n] = tN[n]; }
   }
-  group_sync<64>();
+  group_sync<NT>();
   // per point: traces, averaged Cartesian gradients of the entropy variables
   // and the fluxes (Ismail-Roe, viscous, penalty, symmetrising); the outputs
-  // overwrite T in place when single-pass, else the dead B
+  // overwrite T once every wave has read it
   const double lenScale = fmin(lenE, lenL);
   const double tau = a.tauFact / lenScale;
   // LES length scale of the face: the mean of the two elements'
@@ -255,14 +253,12 @@ __device__ __forceinline__ void face_body(const FaceArgs<K, M, T> &args, const C
   const double lenLES = SGS ? 0.5 * (a.econst[(size_t) e * kElemConst + kElemLenLES]
                                      + a.econst[(size_t) L * kElemConst + kElemLenLES]) : 0.0;
   double evMax = 0.0;
-  for (int m0 = 0; m0 < N2; m0 += G) {
-    const int m = m0 + tid;
-    if (m >= N2) break;
-    const int sp = m / M, fp = m - sp * M;
+  const int sp = m / M, fp = m - sp * M;
+  double Vs[2][5], gx[5], gy[5], gz[5];
+  if (atPoint) {
     T ai[K], di[K];
 #pragma unroll
     for (int sl = 0; sl < K; ++sl) { ai[sl] = sA[sp * K + sl]; di[sl] = sD[sp * K + sl]; }
-    double Vs[2][5], gx[5], gy[5], gz[5];
 #pragma unroll
     for (int v = 0; v < 5; ++v) { gx[v] = 0.0; gy[v] = 0.0; gz[v] = 0.0; }
 #pragma unroll
@@ -270,18 +266,18 @@ __device__ __forceinline__ void face_body(const FaceArgs<K, M, T> &args, const C
       double cm[9];
       if constexpr (!BUG) {
 #pragma unroll
-        for (int q = 0; q < 9; ++q) cm[q] = kGeoEarly ? geoCm[side][q] : g[(side ? 4 + q : 13 + q) * N2 + m];
+        for (int q = 0; q < 9; ++q) cm[q] = geoCm[side][q];
       }
 #pragma unroll
       for (int v = 0; v < 5; ++v) {
-        const T *tA = Tb + side * S::kT1 + v * K * M + fp;
-        const T *tD = tA + 4 * K * M, *tN = tA + 8 * K * M;
+        const T *tA = Tb + side * S::kT1 + v * K * MP + fp;
+        const T *tD = tA + 4 * K * MP, *tN = tA + 8 * K * MP;
         T val = 0, gN = 0, gF = 0, gS = 0;
 #pragma unroll
         for (int sl = 0; sl < K; ++sl) {
-          const T xa = tA[sl * M];
+          const T xa = tA[sl * MP];
           val += ai[sl] * xa;
-          if (v > 0) { gS += di[sl] * xa; gN += ai[sl] * tN[sl * M]; gF += ai[sl] * tD[sl * M]; }
+          if (v > 0) { gS += di[sl] * xa; gN += ai[sl] * tN[sl * MP]; gF += ai[sl] * tD[sl * MP]; }
         }
         Vs[side][v] = kMixed ? double(val) + VCP_FOPS.c03 * sf.Mean[side][v] : double(val);
         if (v == 0) continue;
@@ -301,9 +297,11 @@ __device__ __forceinline__ void face_body(const FaceArgs<K, M, T> &args, const C
     for (int v = 0; v < 5; ++v) asm volatile("" : "+v"(Vs[0][v]), "+v"(Vs[1][v]));
 #pragma unroll
     for (int v = 1; v < 5; ++v) asm volatile("" : "+v"(gx[v]), "+v"(gy[v]), "+v"(gz[v]));
-    const double nn[3] = {kGeoEarly ? geoN[0] : g[0 * N2 + m], kGeoEarly ? geoN[1] : g[1 * N2 + m],
-                          kGeoEarly ? geoN[2] : g[2 * N2 + m]};
-    const double wA = sW2[m] * (kGeoEarly ? geoN[3] : g[3 * N2 + m]);
+  }
+  if constexpr (NT > 64) __syncthreads();
+  if (atPoint) {
+    const double nn[3] = {geoN[0], geoN[1], geoN[2]};
+    const double wA = sW2[m] * geoN[3];
     double fl[5], FX[5], FY[5], FZ[5], ev = 0.0;
     if constexpr (SGS) {
       ev = face_eddy(a.sgs, lenLES, Vs[1], Vs[0], gx, gy, gz);
@@ -311,11 +309,12 @@ __device__ __forceinline__ void face_body(const FaceArgs<K, M, T> &args, const C
     }
     point_flux(Vs[1], Vs[0], gx, gy, gz, nn, wA, tau, a.mu, a.thetaHalf, fl, FX, FY, FZ, 1.0, false, 0.0, nullptr,
                SGS, ev);
+    const int mp = sp * MP + fp;
 #pragma unroll
     for (int v = 0; v < 5; ++v) {
-      sFlux[v * N2 + m] = T(fl[v]);
+      sFlux[v * NP + mp] = T(fl[v]);
       if (v > 0) {
-        sFC[(v - 1) * N2 + m] = T(FX[v]); sFC[(3 + v) * N2 + m] = T(FY[v]); sFC[(7 + v) * N2 + m] = T(FZ[v]);
+        sFC[(v - 1) * NP + mp] = T(FX[v]); sFC[(3 + v) * NP + mp] = T(FY[v]); sFC[(7 + v) * NP + mp] = T(FZ[v]);
       }
     }
   }
@@ -323,23 +322,28 @@ __device__ __forceinline__ void face_body(const FaceArgs<K, M, T> &args, const C
     // the face's eddy-viscosity maximum for the monitoring data
     // (FluxesFace.cpp:336-342)
     evMax = lanes_reduce<G, true>(evMax);
+    if constexpr (NT > 64) {
+      if (tid == 64) sm.EvMax = evMax;
+      __syncthreads();
+      evMax = fmax(evMax, sm.EvMax);
+    }
     if (tid == 0 && live) a.eddyPart[a.nElem + 3 * e + DIR] = evMax;
   }
-  group_sync<64>();
+  group_sync<NT>();
   // ---- lift, one side at a time. Fast-axis lines into Y: the flux (with A)
   // plus the fast slot (with D) of five variables, and the slow and the normal
-  // slot (with A) of variables 1..4; with one face per wave and 9 M <= 64 both
-  // kinds of lines share a pass. Then the slow axis, straight into the face
+  // slot (with A) of variables 1..4; with one face per workgroup and 9 M <= G
+  // both kinds of lines share a pass. Then the slow axis, straight into the face
   // slot of that side: the value plane (A of the first, D of the slow slot)
   // and the normal-derivative plane (A of the normal slot) [0|1][v][slow]
   // [fast]; the volume kernel applies the face vectors.
-  constexpr bool kShare = S::NF == 1 && 9 * M <= 64;
+  constexpr bool kShare = S::NF == 1 && 9 * M <= G;
   static_assert(4 * K <= G || S::NF == 1, "the derivative plane's lines in one pass");
 #pragma unroll
   for (int side = 0; side < 2; ++side) {
     const T sign = side ? T(1) : T(-1);
     double *out = a.faceRes + ((size_t) (side ? L : e) * 6 + 2 * DIR + side) * 10 * K * K;
-    T *Y0 = sf.Y, *YS = sf.Y + 5 * M * K, *YN = YS + 4 * M * K;
+    T *Y0 = sf.X + S::kP, *YS = Y0 + 5 * M * KP, *YN = YS + 4 * M * KP;
     // Cartesian symmetrising flux mapped to this side's parametric slot P
     auto coef = [&](int v, int m, int P, int x) {
       return BUG ? sf.Cm[side][v][3 * P + x] : g[(side ? 4 + 3 * P + x : 13 + 3 * P + x) * N2 + m];
@@ -356,15 +360,15 @@ __device__ __forceinline__ void face_body(const FaceArgs<K, M, T> &args, const C
       T xa[M], xb[M];
 #pragma unroll
       for (int q = 0; q < M; ++q) {
-        const int m = sp * M + q;
-        const double fx = sFC[vc * N2 + m], fy = sFC[(4 + vc) * N2 + m], fz = sFC[(8 + vc) * N2 + m];
+        const int m = sp * M + q, mp = sp * MP + q;
+        const double fx = sFC[vc * NP + mp], fy = sFC[(4 + vc) * NP + mp], fz = sFC[(8 + vc) * NP + mp];
         if constexpr (!BUG)
 #pragma unroll
           for (int x = 0; x < 3; ++x) { cb[x] = coef(vc, m, P0, x); ca[x] = coef(vc, m, PS, x); }
         xb[q] = !isSecond && v == 0 ? T(0) : T(fx * cb[0] + fy * cb[1] + fz * cb[2]);
-        if (!second) xa[q] = sign * sFlux[v * N2 + m];
+        if (!second) xa[q] = sign * sFlux[v * NP + mp];
         else if (!first) xa[q] = T(fx * ca[0] + fy * ca[1] + fz * ca[2]);
-        else xa[q] = isSecond ? T(fx * ca[0] + fy * ca[1] + fz * ca[2]) : sign * sFlux[v * N2 + m];
+        else xa[q] = isSecond ? T(fx * ca[0] + fy * ca[1] + fz * ca[2]) : sign * sFlux[v * NP + mp];
       }
       const auto op = ops();
       const EvenOdd<K, M, T> A = scalar_op<K, M, T>(&op->a);
@@ -377,11 +381,11 @@ __device__ __forceinline__ void face_body(const FaceArgs<K, M, T> &args, const C
         add_modes(scalar_op<K, M, T>(&op->d), xb, z);
         if (!isSecond)
 #pragma unroll
-          for (int n = 0; n < K; ++n) Y0[idx * K + n] = z[n];
+          for (int n = 0; n < K; ++n) Y0[idx * KP + n] = z[n];
       }
       if (second && isSecond)
 #pragma unroll
-        for (int n = 0; n < K; ++n) { YS[idx * K + n] = u[n]; YN[idx * K + n] = w[n]; }
+        for (int n = 0; n < K; ++n) { YS[idx * KP + n] = u[n]; YN[idx * KP + n] = w[n]; }
     };
     if constexpr (kShare) {
       if (tid < 9 * M) lines(tid, true, true, tid >= 5 * M);
@@ -393,16 +397,16 @@ __device__ __forceinline__ void face_body(const FaceArgs<K, M, T> &args, const C
       for (int r = 0; r < (4 * M + G - 1) / G; ++r)
         if (tid + r * G < 4 * M) lines(5 * M + tid + r * G, false, true, true);
     }
-    group_sync<64>();
+    group_sync<NT>();
     // slow-axis lines [0, 5 K) of the value plane, [5 K, 9 K) of the derivative plane
     auto planes = [&](int item, bool first, bool deriv) {
       const int idx = deriv ? item - 5 * K : item, v = deriv ? 1 + idx / K : idx / K, f = idx % K;
-      const T *ya = deriv ? YN + (v - 1) * M * K + f : Y0 + v * M * K + f;
-      const T *yb = YS + (v > 0 ? v - 1 : 0) * M * K + f;
+      const T *ya = deriv ? YN + (v - 1) * M * KP + f : Y0 + v * M * KP + f;
+      const T *yb = YS + (v > 0 ? v - 1 : 0) * M * KP + f;
       const bool slow = !deriv && v > 0;
       T xa[M], xb[M], u[K];
 #pragma unroll
-      for (int q = 0; q < M; ++q) { xa[q] = ya[q * K]; xb[q] = first && slow ? yb[q * K] : T(0); }
+      for (int q = 0; q < M; ++q) { xa[q] = ya[q * KP]; xb[q] = first && slow ? yb[q * KP] : T(0); }
       const auto op = ops();
       to_modes(scalar_op<K, M, T>(&op->a), xa, u);
       if (first) add_modes(scalar_op<K, M, T>(&op->d), xb, u);
@@ -423,7 +427,7 @@ __device__ __forceinline__ void face_body(const FaceArgs<K, M, T> &args, const C
         if (tid + r * G < 5 * K) planes(tid + r * G, true, false);
       if (tid < 4 * K) planes(5 * K + tid, false, true);
     }
-    group_sync<64>();
+    group_sync<NT>();
   }
 #undef VCP_FOPS
 }
@@ -435,7 +439,7 @@ __device__ __forceinline__ void face_body(const FaceArgs<K, M, T> &args, const C
 // form is compiled for two waves per SIMD, where its eddy-viscosity code fits
 // the registers without spilling.
 template <int K, int M, bool BUG, bool BATCH, typename T, bool SGS>
-__global__ __launch_bounds__(64, (SGS ? cmin(2, FaceSmem<K, M, T>::kWaves) : FaceSmem<K, M, T>::kWaves))
+__global__ __launch_bounds__((FaceSmem<K, M, T>::NT), (SGS ? cmin(2, FaceSmem<K, M, T>::kWaves) : FaceSmem<K, M, T>::kWaves))
 void face_kernel(FaceArgs<K, M, T> a_)
 {
   __shared__ FaceSmem<K, M, T> sm;
@@ -479,9 +483,9 @@ void launch_face_kernel(bool bug, int n, FaceArgs<K, M, T> &a, hipStream_t s)
   constexpr int NF = FaceSmem<K, M, T>::NF;
   a.n = n;
   if (bug)
-    hipLaunchKernelGGL((face_kernel<K, M, true, BATCH, T, SGS>), dim3((n + NF - 1) / NF, 3), dim3(64), 0, s, a);
+    hipLaunchKernelGGL((face_kernel<K, M, true, BATCH, T, SGS>), dim3((n + NF - 1) / NF, 3), dim3(FaceSmem<K, M, T>::NT), 0, s, a);
   else
-    hipLaunchKernelGGL((face_kernel<K, M, false, BATCH, T, SGS>), dim3((n + NF - 1) / NF, 3), dim3(64), 0, s, a);
+    hipLaunchKernelGGL((face_kernel<K, M, false, BATCH, T, SGS>), dim3((n + NF - 1) / NF, 3), dim3(FaceSmem<K, M, T>::NT), 0, s, a);
 }
 
 template <int K, int M, typename T>
