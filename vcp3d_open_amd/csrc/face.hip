@@ -43,8 +43,8 @@ struct FaceArgs {
 // all of its lines before it stores over them. LDS regions:
 //   X: normal contraction B -> fast contraction T -> flux and Cartesian
 //      symmetrising fluxes at the points
-//   Y: behind the fluxes in X, the first lift stage of one side: flux + fast
-//      slot of five variables, slow slot and normal slot of variables 1..4
+//   Y: the first lift stage of one side: flux + fast slot of five variables,
+//      slow slot and normal slot of variables 1..4
 //
 // What bounds it: instruction issue and latency at three waves per SIMD (LDS),
 // not memory. The line contractions use the even-odd operators, the lift
@@ -78,7 +78,12 @@ struct FaceSmem {
   static constexpr int KP = K | 1, MP = M | 1, NP = M * MP;
   static constexpr int kB = 2 * 2 * 5 * K * KP, kT1 = 13 * K * MP, kT = 2 * kT1, kP = 17 * NP;
   static constexpr int kY = 13 * M * KP;
-  static constexpr int kX = cmax(cmax(kB, kT), kP + kY);
+  // Y behind the fluxes, over T's end, where that lets one more face into a
+  // CU's LDS and the face is large ((6, 8) 16^3: 110 us, 114 in a region of its
+  // own); at (5, 7) the thirteenth face makes the launch slower (32^3: 554
+  // against 542 us)
+  static constexpr int kOffY = M > 7 ? kP : cmax(cmax(kB, kT), kP);
+  static constexpr int kX = cmax(cmax(kB, kT), kOffY + kY);
   static constexpr int kBytes = (int) sizeof(T) * (2 * M * K + 4 * K + NF * kX) + 8 * (M * M + 1 + NF * 82);
   // waves per SIMD to compile for: three when 12 waves fit a CU's 160 KB
   static constexpr int kWaves = 12 * 64 / NT * kBytes <= 160 * 1024 ? 3 : 2;
@@ -255,7 +260,7 @@ __device__ __forceinline__ void face_body(const FaceArgs<K, M, T> &args, const C
   double evMax = 0.0;
   const int sp = m / M, fp = m - sp * M;
   double Vs[2][5], gx[5], gy[5], gz[5];
-  if (atPoint) {
+  auto traces = [&]() {
     T ai[K], di[K];
 #pragma unroll
     for (int sl = 0; sl < K; ++sl) { ai[sl] = sA[sp * K + sl]; di[sl] = sD[sp * K + sl]; }
@@ -297,9 +302,8 @@ __device__ __forceinline__ void face_body(const FaceArgs<K, M, T> &args, const C
     for (int v = 0; v < 5; ++v) asm volatile("" : "+v"(Vs[0][v]), "+v"(Vs[1][v]));
 #pragma unroll
     for (int v = 1; v < 5; ++v) asm volatile("" : "+v"(gx[v]), "+v"(gy[v]), "+v"(gz[v]));
-  }
-  if constexpr (NT > 64) __syncthreads();
-  if (atPoint) {
+  };
+  auto fluxes = [&]() {
     const double nn[3] = {geoN[0], geoN[1], geoN[2]};
     const double wA = sW2[m] * geoN[3];
     double fl[5], FX[5], FY[5], FZ[5], ev = 0.0;
@@ -317,6 +321,14 @@ __device__ __forceinline__ void face_body(const FaceArgs<K, M, T> &args, const C
         sFC[(v - 1) * NP + mp] = T(FX[v]); sFC[(3 + v) * NP + mp] = T(FY[v]); sFC[(7 + v) * NP + mp] = T(FZ[v]);
       }
     }
+  };
+  if constexpr (NT > 64) {
+    if (atPoint) traces();
+    __syncthreads();
+    if (atPoint) fluxes();
+  } else if (atPoint) {
+    traces();
+    fluxes();
   }
   if (SGS && a.eddyPart) {
     // the face's eddy-viscosity maximum for the monitoring data
@@ -343,7 +355,7 @@ __device__ __forceinline__ void face_body(const FaceArgs<K, M, T> &args, const C
   for (int side = 0; side < 2; ++side) {
     const T sign = side ? T(1) : T(-1);
     double *out = a.faceRes + ((size_t) (side ? L : e) * 6 + 2 * DIR + side) * 10 * K * K;
-    T *Y0 = sf.X + S::kP, *YS = Y0 + 5 * M * KP, *YN = YS + 4 * M * KP;
+    T *Y0 = sf.X + S::kOffY, *YS = Y0 + 5 * M * KP, *YN = YS + 4 * M * KP;
     // Cartesian symmetrising flux mapped to this side's parametric slot P
     auto coef = [&](int v, int m, int P, int x) {
       return BUG ? sf.Cm[side][v][3 * P + x] : g[(side ? 4 + 3 * P + x : 13 + 3 * P + x) * N2 + m];
