@@ -138,7 +138,14 @@ struct ColShape {
   static_assert(H == 1 || LH >= 64, "halves in whole waves");
   // pitches, odd so that lanes a pitch apart fall into different banks
   static constexpr int KP = K | 1, MP = M | 1, NP = N2 | 1;
-  static constexpr int YB = (K * MP) | 1;                // half-transformed lines of one (variable, k)
+  // the planes' lines of one variable, PL apart: at M = 8 a value more than
+  // their length, without which they collide in the banks (16^3 358 / 353 us;
+  // at M = 4 and 6 the gaps cost more, 59 / 57 and 98 / 97 us)
+  static constexpr int PL = M % 8 ? M : M + 1, LP = (M * PL) | 1;
+  // half-transformed lines of one (variable, k): K lines without a gap at
+  // K >= 6 (lines a pitch apart throughout: with a gap of one the 64 lanes of
+  // (6, 8) collide four deep), otherwise an odd number for the reads across them
+  static constexpr int YB = K >= 6 ? K * MP : (K * MP) | 1;
   static constexpr int UV = K * K * KP;                  // one variable of the modal state
   // LDS of one element, in T: B holds the modal state or the lines of the
   // planes of points, X the column coefficients
@@ -148,11 +155,12 @@ struct ColShape {
   // a residual is a difference of large fluxes
   static constexpr int W = (int) (sizeof(double) / sizeof(T));
   static constexpr int X = 5 * K * NP * W;
-  static constexpr int NL = 10 * H * NP;                 // the planes' lines, in double
+  static constexpr int NL = 10 * H * LP;                 // the planes' lines, in double
   static constexpr int B = (cmax(5 * UV, NL * W) + 1) / 2 * 2;
   static constexpr int NY = 5 * K * YB * W;
+  static constexpr int kOther = 8 * (NE * 12 + (G > 64 ? 10 * (G / 64) : 1) + 4 * K + (NE == 1 ? 1 : NE * 45));   // the other LDS arrays
   static constexpr int WGMAX = WAVES * 4 / (NT / 64);    // workgroups per CU by registers
-  static constexpr bool SEPY = (NE * (X + B + NY) * (int) sizeof(T) + 512) * WGMAX <= 160 * 1024;
+  static constexpr bool SEPY = (NE * (X + B + NY) * (int) sizeof(T) + kOther) * WGMAX <= 160 * 1024;
   static constexpr int S = (X + B + (SEPY ? NY : 0) + 1) / 2 * 2;   // whole doubles
   static_assert(NY <= X && 5 * UV <= 5 * K * NP, "the half-transformed lines and A p fit X");
   static constexpr int NDL = (ND + G - 1) / G;           // modes per thread
@@ -326,7 +334,9 @@ void volume_cols_kernel(ColArgs<K, M, T> args_)
   int sp = FULL && a->spIdx ? glob(a->spIdx)[e] : -1;
   if constexpr (kUniform) sp = __builtin_amdgcn_readfirstlane(sp);
   const bool act = tl < N2;
-  const int col = act ? tl : 0, ci = col % M, cj = col / M, colT = ci * M + cj;
+  const int col = act ? tl : 0, ci = col % M, cj = col / M;
+  constexpr int PL = S::PL, LP = S::LP;
+  const int line = cj * PL + ci, lineT = ci * PL + cj;   // its place in the planes' lines along i and j
   const T sgn = T(h ? -1 : 1);
   int half = 0;
   // this thread's points of a column from its coefficients, and back (partial
@@ -479,7 +489,7 @@ void volume_cols_kernel(ColArgs<K, M, T> args_)
   for (int v = 0; v < 5; ++v)
 #pragma unroll
     for (int q = 0; q < K; ++q) acc[v][q] = 0;
-  double *const PB = (double *) B + h * 10 * NP;
+  double *const PB = (double *) B + h * 10 * LP;
   const double w2 = glob(a->tables)[args->oW2 + col];
   const double factHF = a->mu * kGam / kPrLam;
   const double lenLES = FULL && a->sgs ? glob(a->econst)[(size_t) e * kElemConst + kElemLenLES] : 0.0;
@@ -510,7 +520,7 @@ void volume_cols_kernel(ColArgs<K, M, T> args_)
     for (int r = 0; r < (NL + LH - 1) / LH; ++r) {
       const int l = tl + r * LH;
       if (l < NL) {
-        double *x = PB + (l / M) * NP + (l % M) * M;
+        double *x = PB + (l / M) * LP + (l % M) * PL;
         double y[M];
 #pragma unroll
         for (int p = 0; p < M; ++p) y[p] = x[p];
@@ -523,14 +533,17 @@ void volume_cols_kernel(ColArgs<K, M, T> args_)
   // Cartesian gradient of variable v from its parametric derivatives
   auto cartesian = [&](int v, double gr, double gs, double gt, const double (&cur)[kVolGeo], double (&g)[3][5]) {
     cptr<double> vs = (cptr<double>) (uintptr_t) (vg + NI);
+    if (args->bug) {
 #pragma unroll
-    for (int x = 0; x < 3; ++x) {
-      if (!args->bug)
-        g[x][v] = gr * cur[1 + x] + gs * cur[4 + x] + gt * cur[7 + x];
-      else if constexpr (kUniform)
-        g[x][v] = gr * vs[x * NI + v] + gs * vs[(3 + x) * NI + v] + gt * vs[(6 + x) * NI + v];
-      else
-        g[x][v] = gr * sCm[sub][v * 9 + x] + gs * sCm[sub][v * 9 + 3 + x] + gt * sCm[sub][v * 9 + 6 + x];
+      for (int x = 0; x < 3; ++x) {
+        if constexpr (kUniform)
+          g[x][v] = gr * vs[x * NI + v] + gs * vs[(3 + x) * NI + v] + gt * vs[(6 + x) * NI + v];
+        else
+          g[x][v] = gr * sCm[sub][v * 9 + x] + gs * sCm[sub][v * 9 + 3 + x] + gt * sCm[sub][v * 9 + 6 + x];
+      }
+    } else {
+#pragma unroll
+      for (int x = 0; x < 3; ++x) g[x][v] = gr * cur[1 + x] + gs * cur[4 + x] + gt * cur[7 + x];
     }
   };
   // ---------------- sponge, matching-layer and body-force sources, in planes
@@ -554,12 +567,12 @@ void volume_cols_kernel(ColArgs<K, M, T> args_)
         if (cml) {
           if (act)
 #pragma unroll
-            for (int v = 0; v < 5; ++v) { PB[v * NP + tl] = V[v]; PB[(5 + v) * NP + colT] = V[v]; }
+            for (int v = 0; v < 5; ++v) { PB[v * LP + line] = V[v]; PB[(5 + v) * LP + lineT] = V[v]; }
           group_sync<LH>();
           derive_lines(std::integral_constant<int, 10 * M>{}, std::false_type{});
           group_sync<LH>();
 #pragma unroll
-          for (int v = 0; v < 5; ++v) cartesian(v, PB[v * NP + col], PB[(5 + v) * NP + colT], Gt[v], cur, g);
+          for (int v = 0; v < 5; ++v) cartesian(v, PB[v * LP + line], PB[(5 + v) * LP + lineT], Gt[v], cur, g);
         }
         double Vp[5];
 #pragma unroll
@@ -613,13 +626,13 @@ void volume_cols_kernel(ColArgs<K, M, T> args_)
     // lines along i (slots 0..3) and along j (4..7) of variables 1..4
     if (act)
 #pragma unroll
-      for (int v = 0; v < 4; ++v) { PB[v * NP + tl] = V[1 + v]; PB[(4 + v) * NP + colT] = V[1 + v]; }
+      for (int v = 0; v < 4; ++v) { PB[v * LP + line] = V[1 + v]; PB[(4 + v) * LP + lineT] = V[1 + v]; }
     group_sync<LH>();
     derive_lines(std::integral_constant<int, 8 * M>{}, std::false_type{});
     group_sync<LH>();
     double g[3][5];                                   // Cartesian gradients
 #pragma unroll
-    for (int v = 1; v < 5; ++v) cartesian(v, PB[(v - 1) * NP + col], PB[(v + 3) * NP + colT], Gt[v], cur, g);
+    for (int v = 1; v < 5; ++v) cartesian(v, PB[(v - 1) * LP + line], PB[(v + 3) * LP + lineT], Gt[v], cur, g);
     double Ft[5];
     {
       double Fr[5], Fs[5];
@@ -673,7 +686,7 @@ void volume_cols_kernel(ColArgs<K, M, T> args_)
       group_sync<LH>();
       if (act)
 #pragma unroll
-        for (int l = 0; l < 5; ++l) { PB[l * NP + tl] = Fr[l]; PB[(5 + l) * NP + colT] = Fs[l]; }
+        for (int l = 0; l < 5; ++l) { PB[l * LP + line] = Fr[l]; PB[(5 + l) * LP + lineT] = Fs[l]; }
     }
     group_sync<LH>();
     derive_lines(std::integral_constant<int, 10 * M>{}, std::true_type{});
@@ -683,7 +696,7 @@ void volume_cols_kernel(ColArgs<K, M, T> args_)
       cptr<double> Ak = op->Ad + k * K, Dk = op->Dd + k * K;
 #pragma unroll
       for (int v = 0; v < 5; ++v) {
-        const double s = PB[v * NP + col] + PB[(5 + v) * NP + colT];
+        const double s = PB[v * LP + line] + PB[(5 + v) * LP + lineT];
 #pragma unroll
         for (int q = 0; q < K; ++q) {
           acc[v][q] += Ak[q] * s;
