@@ -99,6 +99,10 @@ template <int G>
 __device__ __forceinline__ void group_sync()
 {
   if constexpr (G > 64) {
+    // the wait is written out: at the head of a loop whose body ends with LDS
+    // stores, the compiler (ROCm 7.2, gfx950) leaves it out of the barrier
+    // on the way back
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __syncthreads();
   } else {
     // one wave: its LDS operations complete in order, so only the compiler
