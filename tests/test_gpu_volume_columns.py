@@ -74,8 +74,8 @@ def test_default_follows_the_element_count():
     kernel for a small one, bit for bit."""
     from vcp3d_open_amd.solver import volume_tiles
     for n, which in ((6, 1), (11, 0)):
-        case = TGVCase(n=n, p=2)
-        tiles = volume_tiles(3, 4)
+        case = TGVCase(n=n, p=3)
+        tiles = volume_tiles(4, 5)
         d = evaluate(case, 0, True, "fp64")
         t = evaluate(case, tiles[which], True, "fp64")
         assert np.array_equal(d[2], t[2]) and np.array_equal(d[0], t[0])

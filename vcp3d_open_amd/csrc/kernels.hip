@@ -1171,19 +1171,25 @@ int default_volume_tile(int K, int M)
 // to fill the chip with it: one wave per element (or several elements per
 // wave) runs longer per element than a workgroup, and 256 CUs hold few of
 // them. Measured on one box, volume launch in us, workgroup / column kernel:
-//   (3, 4) 512 elements 30.4 / 35.8, 1728: 44 / 38, 4096: 78 / 48
-//   (4, 5) 512: 36.8 / 44.5, 1000: 43 / 48, 1728: 72 / 64
-//   (4, 6) 512: 42.3 / 46.9, 1000: 58 / 50
-//   (5, 7) 512: 49.7 / 68.3, 1000: 84 / 84, 1728: 116 / 93
-// With two threads per column (K >= 6 in FP64) the column kernel is ahead
-// from the smallest cases on at (6, 8) (27 elements 93 / 81) and once every CU
-// has one at (7, 9) (64: 87 / 90, 216: 85 / 89, 343: 151 / 110); in the float
-// form from a few hundred ((6, 8) 512: 52 / 70, 1000: 84 / 74; (7, 9) 512: 82 / 86).
+//   (4, 5) 512 elements 32.3 / 39.5, 1000: 39.1 / 43.7, 1331: 48.3 / 46.7, 1728: 64 / 53
+//   (4, 6) 512: 36.7 / 41.4, 1000: 68 / 44
+//   (5, 7) 512: 43.7 / 59.3, 1000: 78 / 65, 1728: 100 / 75
+// (4, 6) and (5, 7) hold 768 workgroups at once; the next element costs a
+// second round. With two threads per column (K >= 6 in FP64) the column kernel
+// is ahead from the smallest cases on at (6, 8) (27 elements 76 / 68) and once
+// every CU has one at (7, 9) (216: 73 / 77, 512: 134 / 91); in the float form from
+// a few hundred ((6, 8) 512: 48 / 63, 1000: 87 / 69; (7, 9) 512: 76 / 75).
+// At (3, 4) it is ahead at every size, up to 4096 elements with the columns in
+// halves, when these still run all at once (workgroup / halves / whole:
+// 64 elements 30.0 / 26.0 / 31.7, 1000: 32.3 / 25.4 / 29.9, 4096: 72 / 40 / 43,
+// 5832: 85 / 57 / 49; float 64: 22.8 / 18.3 / 23.1, 4096: 38 / 29 / 32).
 int volume_kind(const DeviceCase &dc, int nt)
 {
-  const int cols = dc.sgs != kSgsNone || dc.nSponge > 0 || dc.fbodyOn ? kVolColsFull : kVolCols;
+  const bool full = dc.sgs != kSgsNone || dc.nSponge > 0 || dc.fbodyOn;
+  const int cols = full ? kVolColsFull : kVolCols;
   if (nt) return nt == default_volume_tile(dc.K, dc.M) ? cols : kVolWorkgroup;
-  const int least = dc.K <= 5 ? 1024 : dc.mixed ? 640 : dc.K == 6 ? 0 : 257;
+  if (dc.K == 3) return dc.nElem > 4096 ? cols : full ? kVolHalvesFull : kVolHalves;
+  const int least = dc.M == 5 ? 1280 : dc.K <= 5 ? 769 : dc.mixed ? 640 : dc.K == 6 ? 0 : 257;
   return dc.nElem >= least ? cols : kVolWorkgroup;
 }
 
@@ -1219,7 +1225,7 @@ hipError_t launch_volume(const DeviceCase &dc, const StageCtl &ctl, hipStream_t 
 {
   const int kind = volume_kind(dc, dc.nt), nt = workgroup_tile(dc.K, dc.M, dc.nt);
   const hipError_t e = [&]() -> hipError_t {
-#define X(k, m) if (kind != kVolWorkgroup && dc.K == k && dc.M == m) return volume_cols<k, m>(dc, kind == kVolColsFull, ctl, s);
+#define X(k, m) if (kind != kVolWorkgroup && dc.K == k && dc.M == m) return volume_cols<k, m>(dc, kind, ctl, s);
     VCP_PAIRS(X)
 #undef X
 #define X(k, m) if (dc.K == k && dc.M == m) return volume_workgroup<k, m>(dc, nt, ctl, s);
@@ -1351,7 +1357,7 @@ hipError_t launch_batch_volume(const BatchGroup &g, int kind, const StageCtl &ct
   const int nt = workgroup_tile(p.K, p.M, g.nt);
 #define X(k, m)                                                                                     \
   if (kind != kVolWorkgroup && p.K == k && p.M == m)                                                \
-    return batch_volume_cols<k, m>(g, kind == kVolColsFull, ctl, w0, nw, s);
+    return batch_volume_cols<k, m>(g, kind, ctl, w0, nw, s);
   VCP_PAIRS(X)
 #undef X
 #define X(k, m) if (p.K == k && p.M == m) return batch_volume_workgroup<k, m>(g, nt, ctl, w0, nw, s);

@@ -190,9 +190,9 @@ hipError_t volume_workgroup(const DeviceCase &dc, int nt, const StageCtl &ctl, h
 template <int K, int M>
 hipError_t batch_volume_workgroup(const BatchGroup &g, int nt, const StageCtl &ctl, int w0, int nw, hipStream_t s);
 template <int K, int M>
-hipError_t volume_cols(const DeviceCase &dc, bool full, const StageCtl &ctl, hipStream_t s);
+hipError_t volume_cols(const DeviceCase &dc, int kind, const StageCtl &ctl, hipStream_t s);
 template <int K, int M>
-hipError_t batch_volume_cols(const BatchGroup &g, bool full, const StageCtl &ctl, int w0, int nw, hipStream_t s);
+hipError_t batch_volume_cols(const BatchGroup &g, int kind, const StageCtl &ctl, int w0, int nw, hipStream_t s);
 hipError_t launch_time_step(const DeviceCase &dc, hipStream_t s);
 // running averages avg = (1 - factNew) avg + factNew q of the current state
 hipError_t launch_average(const DeviceCase &dc, double factNew, hipStream_t s);
@@ -220,8 +220,9 @@ hipError_t launch_batch_faces(const BatchGroup &g, int w0, int nw, hipStream_t s
 hipError_t launch_batch_volume(const BatchGroup &g, int kind, const StageCtl &ctl, int w0, int nw, hipStream_t s);
 // The volume kernel of a case with the given workgroup size (0: the default):
 // volume_kernel, or the column kernel (volume.hip) in its plain form or, for a
-// case with an SGS model, a sponge layer or a body force, its full one.
-enum : int { kVolWorkgroup = 0, kVolCols = 1, kVolColsFull = 2, kVolKinds = 3 };
+// case with an SGS model, a sponge layer or a body force, its full one; at
+// K = 3 for cases of few elements the column kernel with the columns in halves.
+enum : int { kVolWorkgroup = 0, kVolCols = 1, kVolColsFull = 2, kVolHalves = 3, kVolHalvesFull = 4, kVolKinds = 5 };
 int volume_kind(const DeviceCase &dc, int nt);
 // per-element time steps, then per case: the minimum, the synchronization-step
 // clipping into scal[kScalDt], and the step counters; a case with error flags

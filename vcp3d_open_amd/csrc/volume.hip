@@ -116,17 +116,22 @@ __device__ __forceinline__ void group_reduce(double (&v)[NV], double *red, int &
 }
 
 // -------------------------------------------------------------- layout
-template <int K, int M, typename T>
+// Halves of a column in FP64 and float without regard to the number of
+// elements. A column's points are handled by one thread, or by one thread of
+// each half of the group: planes 0 .. (M-1)/2 by the first half, the others,
+// from the last one down, by the second. The whole column in one thread needs a
+// third fewer instructions (the even-odd transforms), but 10 M values and the
+// solve's vectors must fit 256 registers: beyond K = 5 in FP64 they spill ((6, 8)
+// at 16^3: 0.415 ms whole, 0.335 ms halved; (5, 7) at 32^3: 1.04 ms whole, 1.38 ms
+// halved). At K = 3 cases of few elements take halves too (volume_kind): they
+// fill twice as many waves, each with half of the column's serial work.
+template <int K, typename T>
+constexpr int kColHalves = K >= 6 && sizeof(T) == 8 ? 2 : 1;
+
+template <int K, int M, typename T, int HALVES>
 struct ColShape {
   static constexpr int ND = K * K * K, NI = M * M * M, N2 = M * M;
-  // A column's points are handled by one thread (H = 1), or by one thread of
-  // each half of the group (H = 2): planes 0 .. (M-1)/2 by the first half,
-  // the others, from the last one down, by the second. The whole column in
-  // one thread needs a third fewer instructions (the even-odd transforms), but
-  // 10 M values and the solve's vectors must fit 256 registers: beyond K = 5 in
-  // FP64 they spill ((6, 8) at 16^3: 0.415 ms whole, 0.335 ms halved; (5, 7) at
-  // 32^3: 1.04 ms whole, 1.38 ms halved).
-  static constexpr int H = K >= 6 && sizeof(T) == 8 ? 2 : 1;
+  static constexpr int H = HALVES;
   static constexpr int LH = N2 <= 16 ? 16 : N2 <= 32 ? 32 : N2 <= 64 ? 64 : 128;   // threads per half
   static constexpr int G = H * LH;                       // threads per element
   static constexpr int NE = G < 64 ? 64 / G : 1;         // elements per workgroup
@@ -135,7 +140,7 @@ struct ColShape {
   // and runs slower ((4, 5) at 16^3 0.164 against 0.081 ms)
   static constexpr int WAVES = 2;
   static constexpr int HP = H == 1 ? M : (M + 1) / 2;    // planes of a thread (the second half of an odd M: one less)
-  static_assert(H == 1 || LH >= 64, "halves in whole waves");
+  static constexpr bool kInWave = H == 2 && LH < 64;     // the halves share a wave
   // pitches, odd so that lanes a pitch apart fall into different banks
   static constexpr int KP = K | 1, MP = M | 1, NP = N2 | 1;
   // the planes' lines of one variable, PL apart: at M = 8 a value more than
@@ -169,10 +174,9 @@ struct ColShape {
 };
 
 // modal state (pitch KP) -> column coefficients: along i, then along j
-template <int K, int M, typename T>
+template <int K, int M, class S, typename T>
 __device__ __forceinline__ void modes_to_columns(const EvenOdd<K, M, T> &A, const T *u, T *X, T *Y, int t)
 {
-  using S = ColShape<K, M, T>;
 #pragma unroll
   for (int r = 0; r < S::RA; ++r) {
     const int l = t + r * S::G;                          // line (variable k j)
@@ -277,14 +281,15 @@ __device__ __forceinline__ void columns_to_modes(const EvenOdd<K, M, T> &A, T *X
 //          (5, 7) 32^3 1535 / 1042   (6, 8) 16^3 620 / 335   (7, 9) 14^3 720 / 458
 //   float  (3, 4) 60 / 38   (4, 5) 69 / 47   (4, 6) 95 / 52   (5, 7) 1075 / 737
 //          (6, 8) 265 / 209   (7, 9) 385 / 233
-template <int K, int M, bool BATCH, bool FULL, typename T>
-__global__ __launch_bounds__((ColShape<K, M, T>::NT), (ColShape<K, M, T>::WAVES))
+template <int K, int M, bool BATCH, bool FULL, typename T, int HALVES>
+__global__ __launch_bounds__((ColShape<K, M, T, HALVES>::NT), (ColShape<K, M, T, HALVES>::WAVES))
 void volume_cols_kernel(ColArgs<K, M, T> args_)
 {
-  using S = ColShape<K, M, T>;
+  using S = ColShape<K, M, T, HALVES>;
   constexpr bool kMixed = sizeof(T) == 4;
   constexpr int G = S::G, NE = S::NE, ND = S::ND, NI = S::NI, N2 = S::N2, NP = S::NP, H = S::H, HP = S::HP;
   constexpr int LH = S::LH;
+  constexpr bool kInWave = S::kInWave;
   constexpr bool kUniform = NE == 1;            // one element per workgroup
   // a whole column in FP64 fills the registers: the products of the point
   // state stay inside the solve's loop, and its solution is kept in LDS
@@ -302,7 +307,7 @@ void volume_cols_kernel(ColArgs<K, M, T> args_)
   auto ops = [&]() { auto p = &args->op; asm volatile("" : "+s"(p)); return p; };
 
   const int tid = threadIdx.x, sub = G < 64 ? tid / G : 0, t = G < 64 ? tid % G : tid;
-  const int h = H == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid / LH), tl = H == 1 ? t : t - h * LH;
+  const int h = H == 1 ? 0 : kInWave ? t / LH : __builtin_amdgcn_readfirstlane(tid / LH), tl = H == 1 ? t : t - h * LH;
   const int item = blockIdx.x * NE + sub;
   const bool inRange = kUniform || item < args->n;
   // the case part of the arguments: its fields are read where they are used
@@ -338,6 +343,7 @@ void volume_cols_kernel(ColArgs<K, M, T> args_)
   constexpr int PL = S::PL, LP = S::LP;
   const int line = cj * PL + ci, lineT = ci * PL + cj;   // its place in the planes' lines along i and j
   const T sgn = T(h ? -1 : 1);
+  const double sgnD = sgn;
   int half = 0;
   // this thread's points of a column from its coefficients, and back (partial
   // sums over the thread's points): row p of A serves plane p, and with the
@@ -479,7 +485,7 @@ void volume_cols_kernel(ColArgs<K, M, T> args_)
       pr[5] = JacInv * pInv; pr[6] = JacInv * (kGam / kGm1 / rho);
     }
   }
-  modes_to_columns<K, M, T>(scalar_op<K, M, T>(&ops()->a), B, X, Y, t);
+  modes_to_columns<K, M, S, T>(scalar_op<K, M, T>(&ops()->a), B, X, Y, t);
 
   // ---------------- the planes of points: state and gradients, fluxes, and
   // their contraction along k; the in-plane derivatives go through LDS lines
@@ -496,11 +502,16 @@ void volume_cols_kernel(ColArgs<K, M, T> args_)
   const bool cml = FULL && sp >= 0 && a->cml;
   double mach2 = 0.0, evMax = 0.0;
   const int np = H == 1 ? M : h ? M / 2 : (M + 1) / 2;
+  constexpr bool kEqual = LH > 64 || kInWave;      // the halves share barriers or a wave: equal trips
+  // operator rows of plane k: of plane pl, with a change of sign in the odd
+  // modes (of D in the even ones) for the second half, where the halves share
+  // a wave
+  auto row = [&](int pl, int k) { return kInWave ? pl : k; };
   // entropy variables and their derivatives along k at this thread's point of
   // plane k
-  auto plane_values = [&](int k, T (&V)[5], T (&Gt)[5]) {
+  auto plane_values = [&](int rowK, T (&V)[5], T (&Gt)[5]) {
     const auto op = ops();
-    cptr<T> Ak = op->A + k * K, Dk = op->D + k * K;
+    cptr<T> Ak = op->A + rowK * K, Dk = op->D + rowK * K;
 #pragma unroll
     for (int v = 0; v < 5; ++v) {
       T c[K];
@@ -508,7 +519,11 @@ void volume_cols_kernel(ColArgs<K, M, T> args_)
       for (int q = 0; q < K; ++q) c[q] = X[(v * K + q) * NP + col];
       T s = Ak[0] * c[0], d = Dk[1] * c[1];
 #pragma unroll
-      for (int q = 1; q < K; ++q) { s += Ak[q] * c[q]; if (q > 1) d += Dk[q] * c[q]; }
+      for (int q = 1; q < K; ++q) {
+        const T cs = kInWave ? sgn * c[q] : c[q];
+        s += Ak[q] * (q % 2 ? cs : c[q]);
+        if (q > 1) d += Dk[q] * (q % 2 ? c[q] : cs);
+      }
       V[v] = s; Gt[v] = d;
     }
   };
@@ -555,14 +570,14 @@ void volume_cols_kernel(ColArgs<K, M, T> args_)
   if constexpr (FULL)
     if (sp >= 0 || a->bfBuf) {
 #pragma unroll 1
-      for (int pl = 0; pl < (LH > 64 ? HP : np); ++pl) {
-        const bool valid = LH <= 64 || pl < np;
+      for (int pl = 0; pl < (kEqual ? HP : np); ++pl) {
+        const bool valid = !kEqual || pl < np;
         const int k = H == 2 && h ? M - 1 - pl : pl, m = k * N2 + col;
         double cur[kVolGeo];
 #pragma unroll
         for (int q = 0; q < kVolGeo; ++q) cur[q] = vg[(unsigned) (q * NI + m)];
         T V[5], Gt[5];
-        plane_values(k, V, Gt);
+        plane_values(row(pl, k), V, Gt);
         double g[3][5];
         if (cml) {
           if (act)
@@ -578,7 +593,7 @@ void volume_cols_kernel(ColArgs<K, M, T> args_)
 #pragma unroll
         for (int v = 0; v < 5; ++v) Vp[v] = double(V[v]) + meanPt[v];
         const EntState st = ent_state(Vp);
-        const double wJ = w2 * args->op.w[k] * cur[0], weight = -wJ;
+        const double wJ = w2 * args->op.w[row(pl, k)] * cur[0], weight = -wJ;
         double src[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
         if (sp >= 0) {
           // sponge damping sigma J w (U - U_target) and CML sources
@@ -605,24 +620,24 @@ void volume_cols_kernel(ColArgs<K, M, T> args_)
           src[4] += weight * (st.u * bx + st.v * by + st.w * bz);
         }
         if (valid) {
-          cptr<double> Ak = ops()->Ad + k * K;
+          cptr<double> Ak = ops()->Ad + row(pl, k) * K;
 #pragma unroll
           for (int v = 0; v < 5; ++v)
 #pragma unroll
-            for (int q = 0; q < K; ++q) acc[v][q] += Ak[q] * src[v];
+            for (int q = 0; q < K; ++q) acc[v][q] += Ak[q] * (kInWave && q % 2 ? sgnD * src[v] : src[v]);
         }
         group_sync<LH>();
       }
     }
 #pragma unroll 1
-  for (int pl = 0; pl < (LH > 64 ? HP : np); ++pl) {
-    const bool valid = LH <= 64 || pl < np;      // equal trips where the halves share barriers
+  for (int pl = 0; pl < (kEqual ? HP : np); ++pl) {
+    const bool valid = !kEqual || pl < np;
     const int k = H == 2 && h ? M - 1 - pl : pl;
     double cur[kVolGeo];
 #pragma unroll
     for (int q = 0; q < kVolGeo; ++q) cur[q] = vg[(unsigned) (q * NI + k * N2 + col)];
     T V[5], Gt[5];
-    plane_values(k, V, Gt);
+    plane_values(row(pl, k), V, Gt);
     // lines along i (slots 0..3) and along j (4..7) of variables 1..4
     if (act)
 #pragma unroll
@@ -668,7 +683,7 @@ void volume_cols_kernel(ColArgs<K, M, T> args_)
       const double fx[5] = {ru, ru * u - txx + p, rv * u - txy, rw * u - txz, (rE + p) * u - (u * txx + v * txy + w * txz - qx)};
       const double fy[5] = {rv, ru * v - txy, rv * v - tyy + p, rw * v - tyz, (rE + p) * v - (u * txy + v * tyy + w * tyz - qy)};
       const double fz[5] = {rw, ru * w - txz, rv * w - tyz, rw * w - tzz + p, (rE + p) * w - (u * txz + v * tyz + w * tzz - qz)};
-      const double wJ = w2 * args->op.w[k] * cur[0], weight = -wJ;
+      const double wJ = w2 * args->op.w[row(pl, k)] * cur[0], weight = -wJ;
 #pragma unroll
       for (int d = 0; d < 3; ++d) {
         const double mx = weight * cur[1 + 3 * d], my = weight * cur[2 + 3 * d], mz = weight * cur[3 + 3 * d];
@@ -693,14 +708,14 @@ void volume_cols_kernel(ColArgs<K, M, T> args_)
     group_sync<LH>();
     if (valid) {
       const auto op = ops();
-      cptr<double> Ak = op->Ad + k * K, Dk = op->Dd + k * K;
+      cptr<double> Ak = op->Ad + row(pl, k) * K, Dk = op->Dd + row(pl, k) * K;
 #pragma unroll
       for (int v = 0; v < 5; ++v) {
         const double s = PB[v * LP + line] + PB[(5 + v) * LP + lineT];
 #pragma unroll
         for (int q = 0; q < K; ++q) {
-          acc[v][q] += Ak[q] * s;
-          if (q > 0) acc[v][q] += Dk[q] * Ft[v];
+          acc[v][q] += Ak[q] * (kInWave && q % 2 ? sgnD * s : s);
+          if (q > 0) acc[v][q] += Dk[q] * (kInWave && q % 2 == 0 ? sgnD * Ft[v] : Ft[v]);
         }
       }
     }
@@ -847,7 +862,7 @@ void volume_cols_kernel(ColArgs<K, M, T> args_)
         break;
       }
       group_sync<G>();
-      modes_to_columns(A, B, X, Y, t);
+      modes_to_columns<K, M, S, T>(A, B, X, Y, t);
       {
         T y[5][HP];
 #pragma unroll
@@ -1007,44 +1022,53 @@ void fill_col_args(const DeviceCase &dc, const StageCtl &ctl, ColArgs<K, M, T> &
   a.op.c03 = dc.opC0[0] * dc.opC0[0] * dc.opC0[0];
 }
 
-template <int K, int M, bool BATCH, typename T>
-hipError_t launch_cols(const DeviceCase &dc, bool full, ColArgs<K, M, T> &a, hipStream_t s)
+template <int K, int M, bool BATCH, int HALVES, typename T>
+hipError_t launch_cols(bool full, ColArgs<K, M, T> &a, hipStream_t s)
 {
-  using S = ColShape<K, M, T>;
+  using S = ColShape<K, M, T, HALVES>;
   const dim3 grid((a.n + S::NE - 1) / S::NE), block(S::NT);
-  if (full) hipLaunchKernelGGL((volume_cols_kernel<K, M, BATCH, true, T>), grid, block, 0, s, a);
-  else hipLaunchKernelGGL((volume_cols_kernel<K, M, BATCH, false, T>), grid, block, 0, s, a);
+  if (full) hipLaunchKernelGGL((volume_cols_kernel<K, M, BATCH, true, T, HALVES>), grid, block, 0, s, a);
+  else hipLaunchKernelGGL((volume_cols_kernel<K, M, BATCH, false, T, HALVES>), grid, block, 0, s, a);
   return hipGetLastError();
+}
+
+template <int K, int M, bool BATCH, typename T>
+hipError_t launch_kind(int kind, ColArgs<K, M, T> &a, hipStream_t s)
+{
+  const bool full = kind == kVolColsFull || kind == kVolHalvesFull;
+  if constexpr (K == 3)
+    if (kind == kVolHalves || kind == kVolHalvesFull) return launch_cols<K, M, BATCH, 2>(full, a, s);
+  return launch_cols<K, M, BATCH, kColHalves<K, T>>(full, a, s);
 }
 
 }  // namespace
 
 template <int K, int M>
-hipError_t volume_cols(const DeviceCase &dc, bool full, const StageCtl &ctl, hipStream_t s)
+hipError_t volume_cols(const DeviceCase &dc, int kind, const StageCtl &ctl, hipStream_t s)
 {
   auto run = [&](auto zero) {
     ColArgs<K, M, decltype(zero)> a{};
     a.c = case_dev(dc); a.n = dc.nElem;
     fill_col_args(dc, ctl, a);
-    return launch_cols<K, M, false>(dc, full, a, s);
+    return launch_kind<K, M, false>(kind, a, s);
   };
   return dc.mixed ? run(0.0f) : run(0.0);
 }
 
 template <int K, int M>
-hipError_t batch_volume_cols(const BatchGroup &g, bool full, const StageCtl &ctl, int w0, int nw, hipStream_t s)
+hipError_t batch_volume_cols(const BatchGroup &g, int kind, const StageCtl &ctl, int w0, int nw, hipStream_t s)
 {
   auto run = [&](auto zero) {
     ColArgs<K, M, decltype(zero)> a{};
     a.cases = g.cases; a.work = g.work; a.w0 = w0; a.n = nw;
     fill_col_args(*g.proto, ctl, a);
-    return launch_cols<K, M, true>(*g.proto, full, a, s);
+    return launch_kind<K, M, true>(kind, a, s);
   };
   return g.proto->mixed ? run(0.0f) : run(0.0);
 }
 
-template hipError_t volume_cols<VCP_SHAPE_K, VCP_SHAPE_M>(const DeviceCase &, bool, const StageCtl &, hipStream_t);
-template hipError_t batch_volume_cols<VCP_SHAPE_K, VCP_SHAPE_M>(const BatchGroup &, bool, const StageCtl &, int, int,
+template hipError_t volume_cols<VCP_SHAPE_K, VCP_SHAPE_M>(const DeviceCase &, int, const StageCtl &, hipStream_t);
+template hipError_t batch_volume_cols<VCP_SHAPE_K, VCP_SHAPE_M>(const BatchGroup &, int, const StageCtl &, int, int,
                                                                 hipStream_t);
 
 }  // namespace vcp
