@@ -6,10 +6,14 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <memory>
+#include <mutex>
 #include <string>
+#include <system_error>
+#include <thread>
 #include <utility>
 #include <vector>
 
@@ -25,6 +29,16 @@ int fail(const std::string &msg, int code)
   return code;
 }
 
+std::shared_ptr<Staging> Staging::shared()
+{
+  static std::mutex m;
+  static std::weak_ptr<Staging> current;
+  std::lock_guard<std::mutex> lock(m);
+  std::shared_ptr<Staging> s = current.lock();
+  if (!s) current = s = std::make_shared<Staging>();
+  return s;
+}
+
 }  // namespace vcp
 
 using vcp::fail;
@@ -36,6 +50,73 @@ namespace {
 constexpr int kScalRead = vcp::kScalEddy + 1, kHostFlags = vcp::kScalCount;
 
 size_t state_size(const vcp_ctx *c) { return (size_t) c->dc.nElem * 5 * c->dc.nDOF; }
+
+// Waits for the context's stream and reads n doubles of device memory back into
+// the caller's (pageable) array. The runtime copies into pageable memory at 17
+// GB/s at best and takes the page faults of a new array besides, all on one
+// thread; through pinned chunks the copy runs at the link's 57 GB/s, and several
+// threads move the chunks and share the faults. From 16 MB on, where that
+// outweighs starting the threads: 164 MB into a
+// new array 15.2 ms directly, 4.4 ms staged; 35 MB 2.4 / 1.3 ms, 18 MB 1.3 / 0.9 ms.
+int read_back(vcp_ctx *c, double *dst, const double *src, size_t n)
+{
+  using vcp::Staging;
+  const size_t bytes = n * sizeof(double);
+  Staging &st = *c->staging;
+  std::unique_lock<std::mutex> lock(st.taken, std::defer_lock);
+  bool staged = bytes >= 8 * Staging::kChunk && lock.try_lock();
+  if (staged && !st.buf
+      && hipHostMalloc((void **) &st.buf, 2 * Staging::kThreads * Staging::kChunk, hipHostMallocDefault) != hipSuccess) {
+    (void) hipGetLastError();
+    st.buf = nullptr;
+    staged = false;
+  }
+  if (!staged) {
+    HIP_TRY(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, c->stream));
+    HIP_TRY(hipStreamSynchronize(c->stream));
+    return 0;
+  }
+  int device = 0;
+  HIP_TRY(hipGetDevice(&device));
+  vcp::EventSet es;
+  HIP_TRY(es.create(2 * Staging::kThreads));
+  const size_t chunks = (bytes + Staging::kChunk - 1) / Staging::kChunk;
+  hipError_t err[Staging::kThreads] = {};
+  // thread t moves the chunks t, t + kThreads, ... through its two pinned
+  // chunks: the next one is on its way while it copies the last
+  auto move = [&](int t) {
+    hipError_t he = hipSetDevice(device);
+    auto size = [&](size_t k) { return std::min(Staging::kChunk, bytes - k * Staging::kChunk); };
+    auto slot = [&](size_t i) { return st.buf + (2 * t + i % 2) * Staging::kChunk; };
+    auto start = [&](size_t k, size_t i) {
+      if (he == hipSuccess && k < chunks) {
+        he = hipMemcpyAsync(slot(i), (const char *) src + k * Staging::kChunk, size(k), hipMemcpyDeviceToHost, c->stream);
+        if (he == hipSuccess) he = hipEventRecord(es.ev[2 * t + i % 2], c->stream);
+      }
+    };
+    start(t, 0);
+    size_t i = 0;
+    for (size_t k = t; k < chunks && he == hipSuccess; k += Staging::kThreads, ++i) {
+      start(k + Staging::kThreads, i + 1);
+      if (he == hipSuccess) he = hipEventSynchronize(es.ev[2 * t + i % 2]);
+      if (he == hipSuccess) std::memcpy((char *) dst + k * Staging::kChunk, slot(i), size(k));
+    }
+    err[t] = he;
+  };
+  std::vector<std::thread> pool;
+  pool.reserve(Staging::kThreads);
+  int t = 1;
+  try {
+    for (; t < Staging::kThreads; ++t) pool.emplace_back(move, t);
+  } catch (const std::system_error &) {
+  }
+  move(0);
+  for (; t < Staging::kThreads; ++t) move(t);     // threads that could not be started
+  for (std::thread &th : pool) th.join();
+  HIP_TRY(hipStreamSynchronize(c->stream));       // no copy is left in the pinned chunks
+  for (hipError_t e : err) HIP_TRY(e);
+  return 0;
+}
 
 int flag_error(int flags)
 {
@@ -582,9 +663,7 @@ int vcp_get_solution(vcp_ctx *c, double *modal)
   VCP_GUARD_BEGIN
   if (!c || !modal) return fail("null argument");
   if (int rc_ = vcp::batch_quiesce(c)) return rc_;
-  HIP_TRY(hipMemcpyAsync(modal, c->dc.U, state_size(c) * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-  HIP_TRY(hipStreamSynchronize(c->stream));
-  return 0;
+  return read_back(c, modal, c->dc.U, state_size(c));
   VCP_GUARD_END
 }
 
@@ -609,9 +688,7 @@ int vcp_get_residual(vcp_ctx *c, double *modal)
   VCP_GUARD_BEGIN
   if (!c || !modal) return fail("null argument");
   if (int rc_ = vcp::batch_quiesce(c)) return rc_;
-  HIP_TRY(hipMemcpyAsync(modal, c->dc.R, state_size(c) * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-  HIP_TRY(hipStreamSynchronize(c->stream));
-  return 0;
+  return read_back(c, modal, c->dc.R, state_size(c));
   VCP_GUARD_END
 }
 

@@ -7,6 +7,7 @@
 
 #include <exception>
 #include <memory>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -37,7 +38,28 @@ int fail(const std::string &msg, int code = -1);
   catch (const std::exception &ex_) { return vcp::fail(std::string("exception: ") + ex_.what(), -2); } \
   catch (...) { return vcp::fail("unknown exception", -2); }
 
+namespace vcp {
+
+// Pinned host memory that large states are read back through, one for all
+// contexts of the process: allocated on the first large readback, freed with
+// the last context. Whoever finds it taken by another thread reads back
+// without it.
+struct Staging {
+  static constexpr size_t kChunk = size_t(2) << 20;      // bytes per copy
+  static constexpr int kThreads = 8;                     // host threads, two chunks each
+  std::mutex taken;
+  char *buf = nullptr;
+  ~Staging()
+  {
+    if (buf) (void) hipHostFree(buf);
+  }
+  static std::shared_ptr<Staging> shared();
+};
+
+}  // namespace vcp
+
 struct vcp_ctx {
+  std::shared_ptr<vcp::Staging> staging = vcp::Staging::shared();
   vcp::CaseParams prm;
   vcp::Tables tab;
   vcp::RefConditions rc{};
