@@ -1071,6 +1071,20 @@ __global__ void fill_kernel(double *p, size_t n, double v)
 
 // The time step of the RK step about to run, into device memory (one lane,
 // a vector store).
+__global__ __launch_bounds__(64) void publish_kernel(const double *scal, const int *flags, double *host, int n,
+                                                     int flagsAt)
+{
+  const int i = threadIdx.x;
+  if (i < n) host[i] = scal[i];
+  if (i == 0) *(int *) (host + flagsAt) = flags[kWordFlags];
+}
+
+__global__ __launch_bounds__(256) void store_kernel(double *dst, const double *src, size_t n)
+{
+  const size_t i = (size_t) blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) dst[i] = src[i];
+}
+
 __global__ void set_dt_kernel(double *p, double v)
 {
   if (threadIdx.x == 0) *p = v;
@@ -1323,6 +1337,20 @@ hipError_t static_scratch(void **ptr, size_t *bytes)
   *ptr = addr[dev];
   *bytes = sizeof(scratch);
   return hipSuccess;
+}
+
+hipError_t launch_publish(const DeviceCase &dc, double *host, int n, int flagsAt, hipStream_t s)
+{
+  if (n > 64) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(publish_kernel, dim3(1), dim3(64), 0, s, dc.scal, dc.flags, host, n, flagsAt);
+  return hipGetLastError();
+}
+
+hipError_t launch_store(double *dst, const double *src, size_t n, hipStream_t s)
+{
+  if (n == 0) return hipSuccess;
+  hipLaunchKernelGGL(store_kernel, dim3((unsigned) ((n + 255) / 256)), dim3(256), 0, s, dst, src, n);
+  return hipGetLastError();
 }
 
 hipError_t launch_set_dt(const DeviceCase &dc, double dt, hipStream_t s)

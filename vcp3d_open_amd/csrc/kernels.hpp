@@ -201,6 +201,11 @@ hipError_t launch_average(const DeviceCase &dc, double factNew, hipStream_t s);
 hipError_t launch_damping_from_averages(const DeviceCase &dc, hipStream_t s);
 // scal[kScalDt] = dt, ordered on the stream
 hipError_t launch_set_dt(const DeviceCase &dc, double dt, hipStream_t s);
+// host[0, n) = the device scalars, host[flagsAt] = the error flags (as int);
+// host: pinned memory, valid after a wait for the stream
+hipError_t launch_publish(const DeviceCase &dc, double *host, int n, int flagsAt, hipStream_t s);
+// dst[0, n) = src[0, n); dst may be pinned host memory
+hipError_t launch_store(double *dst, const double *src, size_t n, hipStream_t s);
 // p[0, n) = v on stream s
 hipError_t launch_fill(double *p, size_t n, double v, hipStream_t s);
 // The library's fixed device scratch array (64 MiB per device, held until the
