@@ -239,7 +239,7 @@ def bench_batch(args) -> int:
     attainable = min(PEAK_FP64_TFLOPS, PEAK_HBM_GBS * intensity / 1e3)
     roofline = {"bound": "valu-fp64" if attainable >= PEAK_FP64_TFLOPS else "hbm", "achieved": achieved,
                 "peak": PEAK_FP64_TFLOPS, "unit": "TFLOP/s", "frac": achieved / PEAK_FP64_TFLOPS,
-                "traffic": None, "kernel": f"volume_kernel<{K}, {M}, {top['volume_threads']}, batch>",
+                "traffic": None, "kernel": f"volume kernels of ({K}, {M}), batch",
                 "ms_per_launch": ms, "algorithmic_flops": flops, "algorithmic_bytes": bytes_,
                 "intensity_flop_per_byte": intensity, "attainable_tflops": attainable,
                 "frac_of_attainable": achieved / attainable, "groups": per_group}
@@ -516,7 +516,7 @@ def main() -> int:
     rs_face, rs_vol = solver.profile_residual(args.profile_reps)
     K, M = case.p + 1, 7
     if ms_vol >= ms_face:
-        name, ms = "volume_kernel<5, 7, 256>", ms_vol
+        name, ms = "volume_cols_kernel<5, 7>", ms_vol
         flops = volume_kernel_flops(K, M, cg_mean) * case.n_elems
         bytes_ = volume_kernel_bytes(K, M, 2.0 / 3.0) * case.n_elems
     else:
