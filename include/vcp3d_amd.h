@@ -270,7 +270,8 @@ int vcp_profile_residual(vcp_ctx *ctx, int reps, double ms[2]);
    of integration points, named by its threads per plane of points), the
    others are workgroups of that many threads. The default is the column
    kernel for cases large enough to fill the chip with it and the second size
-   for smaller ones. Results of different sizes agree to rounding (partial sums
+   for smaller ones; at nDOFs1D = 3 it is the column kernel throughout, with two
+   threads per column up to 4096 elements. Results of different sizes agree to rounding (partial sums
    are grouped differently); a given size gives identical results every run. */
 int vcp_set_tile(vcp_ctx *ctx, int nt);
 
