@@ -1,0 +1,62 @@
+"""Host code of the library (contexts, batches, readbacks) on a stand-in for the
+HIP runtime (hip_host.cpp): no GPU, kernels recorded and not run. Each test is a
+process of its own, so that the stand-in never meets the real runtime."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+ROOT = os.path.dirname(HERE)
+
+PRELUDE = """
+import ctypes, sys
+import numpy as np
+rt = ctypes.CDLL({lib!r}, mode=ctypes.RTLD_GLOBAL)
+rt.rt_launches.restype = ctypes.c_char_p
+rt.rt_fail_new.argtypes = [ctypes.c_long]
+from vcp3d_open_amd.cases import OpenBoxCase, TGVCase
+from vcp3d_open_amd.solver import Batch, SolverClass, VCPError
+
+def launches(kernel):
+    return [line for line in rt.rt_launches().decode().splitlines() if kernel in line]
+
+def solver(precision="fp64", **kw):
+    s = SolverClass(TGVCase(**kw), precision=precision)
+    s.ReadRestartSolution(TGVCase(**kw).initial_conservative())
+    return s
+"""
+
+
+@pytest.fixture(scope="session")
+def host_runtime(tmp_path_factory):
+    lib = str(tmp_path_factory.mktemp("hip_host") / "libhip_host.so")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", "-o", lib, os.path.join(HERE, "hip_host.cpp")],
+                   check=True)
+
+    def run(script):
+        p = subprocess.run([sys.executable, "-c", PRELUDE.format(lib=lib) + script], cwd=ROOT, capture_output=True,
+                           text=True, timeout=120)
+        assert p.returncode == 0, f"exit {p.returncode}\n{p.stdout}\n{p.stderr}"
+        return p.stdout
+
+    return run
+
+
+def test_batch_whose_group_was_emptied(host_runtime):
+    """A group that has lost its last case launches nothing: not in a profile,
+    which visits every group, and not in a step."""
+    host_runtime("""
+a, b = solver(n=3, p=2), solver(n=3, p=3)
+batch = Batch()
+batch.add(a); batch.add(b)
+batch.step(1); batch.wait()
+batch.remove(a)
+rt.rt_clear()
+assert len(batch.profile(1)) == 2
+assert not launches("_kernel<3,")
+assert len(launches("volume")) == 1
+batch.step(1); batch.wait()
+assert not launches("_kernel<3,")
+""")

@@ -18,6 +18,7 @@
 #include <algorithm>
 #include <climits>
 #include <cstring>
+#include <iterator>
 
 using vcp::fail;
 
@@ -123,6 +124,7 @@ int upload(vcp_batch *b)
       g.first.push_back((int) work.size());
     }
     g.nWork = (int) work.size();
+    std::fill(std::begin(g.kind), std::end(g.kind), 0);   // a group without cases launches nothing
     if (g.cases.empty()) continue;
     if (!g.stream) HIP_TRY(hipStreamCreate(&g.stream));
     if (!g.done) HIP_TRY(hipEventCreateWithFlags(&g.done, hipEventDisableTiming));
