@@ -60,3 +60,19 @@ assert len(launches("volume")) == 1
 batch.step(1); batch.wait()
 assert not launches("_kernel<3,")
 """)
+
+
+# 1.1 KB (a kernel's stores), 1.1 MB (one copy) and 18 MB (chunks on several threads)
+@pytest.mark.parametrize("n,p", [(2, 2), (6, 4), (15, 4)])
+def test_read_back_on_another_current_device(host_runtime, n, p):
+    """A host thread whose current device is not the context's reads its
+    states, as it sets them, and keeps its current device."""
+    host_runtime(f"""
+s = solver(n={n}, p={p})
+u = np.random.default_rng(1).standard_normal((s.n_elem, 5, s.n_dofs))
+rt.rt_set_device(1)
+s.set_solution(u)
+assert np.array_equal(s.solution(), u)
+s.residual_array()
+assert rt.rt_device() == 1
+""")

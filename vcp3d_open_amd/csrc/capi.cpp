@@ -64,6 +64,8 @@ int read_back(vcp_ctx *c, double *dst, const double *src, size_t n)
 {
   using vcp::Staging;
   const size_t bytes = n * sizeof(double);
+  vcp::DeviceScope scope;
+  HIP_TRY(scope.enter(c->device));
   if (n <= (size_t) kSmallState) {
     // up to 128 KB a kernel writes it into the context's pinned words
     HIP_TRY(vcp::launch_store(c->host + kHostState, src, n, c->stream));
@@ -85,8 +87,6 @@ int read_back(vcp_ctx *c, double *dst, const double *src, size_t n)
     HIP_TRY(hipStreamSynchronize(c->stream));
     return 0;
   }
-  int device = 0;
-  HIP_TRY(hipGetDevice(&device));
   vcp::EventSet es;
   HIP_TRY(es.create(2 * Staging::kThreads));
   const size_t chunks = (bytes + Staging::kChunk - 1) / Staging::kChunk;
@@ -94,7 +94,7 @@ int read_back(vcp_ctx *c, double *dst, const double *src, size_t n)
   // thread t moves the chunks t, t + kThreads, ... through its two pinned
   // chunks: the next one is on its way while it copies the last
   auto move = [&](int t) {
-    hipError_t he = hipSetDevice(device);
+    hipError_t he = hipSetDevice(c->device);
     auto size = [&](size_t k) { return std::min(Staging::kChunk, bytes - k * Staging::kChunk); };
     auto slot = [&](size_t i) { return st.buf + (2 * t + i % 2) * Staging::kChunk; };
     auto start = [&](size_t k, size_t i) {
@@ -454,7 +454,8 @@ int vcp_create(const vcp_case_desc *d, const double *elem_grid, vcp_ctx **out)
   const int nInt = dc.nInt, n2 = dc.nInt2D;
   const size_t nVgeo = (size_t) nElem * vcp::kVolGeo * nInt, nFgeo = (size_t) nElem * 3 * vcp::kFaceGeo * n2;
   const size_t nEcon = (size_t) nElem * vcp::kElemConst;
-  hipError_t he = hipStreamCreate(&c->stream);
+  hipError_t he = hipGetDevice(&c->device);
+  if (he == hipSuccess) he = hipStreamCreate(&c->stream);
   if (he == hipSuccess) he = hipHostMalloc((void **) &c->host, (kHostState + kSmallState) * sizeof(double), hipHostMallocDefault);
   if (he == hipSuccess) he = hipStreamCreate(&c->side);
   if (he == hipSuccess) he = hipEventCreateWithFlags(&c->evState, hipEventDisableTiming);

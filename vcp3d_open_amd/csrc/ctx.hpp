@@ -59,6 +59,7 @@ struct Staging {
 }  // namespace vcp
 
 struct vcp_ctx {
+  int device = 0;                 // the current device at creation, which holds everything below
   std::shared_ptr<vcp::Staging> staging = vcp::Staging::shared();
   vcp::CaseParams prm;
   vcp::Tables tab;
@@ -152,6 +153,26 @@ struct EventSet {
   {
     for (hipEvent_t e : ev)
       if (e) (void) hipEventDestroy(e);
+  }
+};
+
+// Makes a device the calling thread's current one for its lifetime: events and
+// kernel launches take the current device, which has to be their stream's.
+struct DeviceScope {
+  int before = 0;
+  bool switched = false;
+  hipError_t enter(int device)
+  {
+    hipError_t e = hipGetDevice(&before);
+    if (e == hipSuccess && before != device) {
+      e = hipSetDevice(device);
+      switched = e == hipSuccess;
+    }
+    return e;
+  }
+  ~DeviceScope()
+  {
+    if (switched) (void) hipSetDevice(before);
   }
 };
 
