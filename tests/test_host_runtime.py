@@ -76,3 +76,22 @@ assert np.array_equal(s.solution(), u)
 s.residual_array()
 assert rt.rt_device() == 1
 """)
+
+
+def test_staged_read_back_without_memory_for_its_threads(host_runtime):
+    """An allocation that fails anywhere in a staged readback, also while its
+    threads are being started, is an error of that call or none at all; the
+    process goes on and the next readback is whole."""
+    host_runtime("""
+s = solver(n=15, p=4)
+u = np.random.default_rng(1).standard_normal((s.n_elem, 5, s.n_dofs))
+s.set_solution(u)
+out = np.zeros_like(u)
+for after in range(14):
+    out[:] = 0.0
+    rt.rt_fail_new(after)
+    rc = s._L.vcp_get_solution(s.h, out)
+    rt.rt_fail_new(-1)
+    assert rc < 0 or np.array_equal(out, u)
+    assert np.array_equal(s.solution(), u)
+""")

@@ -9,10 +9,10 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <exception>
 #include <memory>
 #include <mutex>
 #include <string>
-#include <system_error>
 #include <thread>
 #include <utility>
 #include <vector>
@@ -117,7 +117,7 @@ int read_back(vcp_ctx *c, double *dst, const double *src, size_t n)
   int t = 1;
   try {
     for (; t < Staging::kThreads; ++t) pool.emplace_back(move, t);
-  } catch (const std::system_error &) {
+  } catch (const std::exception &) {              // no thread or no memory for one
   }
   move(0);
   for (; t < Staging::kThreads; ++t) move(t);     // threads that could not be started
