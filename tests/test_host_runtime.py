@@ -95,3 +95,23 @@ for after in range(14):
     assert rc < 0 or np.array_equal(out, u)
     assert np.array_equal(s.solution(), u)
 """)
+
+
+def test_cases_joining_a_batch_share_their_first_launches(host_runtime):
+    """The first residual of the cases that join a batch takes one volume launch
+    per kernel among them, however many they are."""
+    host_runtime("""
+batch = Batch()
+running = solver(n=3, p=3)
+batch.add(running)
+batch.step(1)
+late = [solver(n=3, p=3), solver(n=11, p=3), solver(n=4, p=3)]
+for s in late:
+    batch.add(s)
+rt.rt_clear()
+batch.step(0)
+elements = sorted(int(line.split()[-1]) for line in launches("volume"))
+# (4, 5): one workgroup per element of the small cases, one of the column kernel per two of the large one
+assert elements == [27 + 64, (1331 + 1) // 2], launches("volume")
+assert len(launches("face")) == 1
+""")

@@ -34,6 +34,7 @@ struct vcp_batch {
     vcp::WorkItem *dWorkV = nullptr;   // the items ordered by volume kernel
     size_t capWorkV = 0;
     int kind[vcp::kVolKinds + 1] = {}; // first item of each kernel in dWorkV
+    std::vector<int> caseKind;         // the kernel of each case
     int *dStatus = nullptr;
     int nWork = 0;
     int initFrom = -1;                 // cases [initFrom, end) need their first residual
@@ -140,10 +141,12 @@ int upload(vcp_batch *b)
     HIP_TRY(hipMemcpy(g.dWork, work.data(), work.size() * sizeof(vcp::WorkItem), hipMemcpyHostToDevice));
     std::vector<vcp::WorkItem> workV;
     workV.reserve(work.size());
+    g.caseKind.clear();
+    for (const vcp_ctx *c : g.cases) g.caseKind.push_back(vcp::volume_kind(c->dc, g.nt));
     for (int k = 0; k < vcp::kVolKinds; ++k) {
       g.kind[k] = (int) workV.size();
       for (size_t ci = 0; ci < g.cases.size(); ++ci)
-        if (vcp::volume_kind(g.cases[ci]->dc, g.nt) == k)
+        if (g.caseKind[ci] == k)
           workV.insert(workV.end(), work.begin() + g.first[ci], work.begin() + g.first[ci + 1]);
     }
     g.kind[vcp::kVolKinds] = (int) workV.size();
@@ -154,14 +157,19 @@ int upload(vcp_batch *b)
   return 0;
 }
 
-// Volume launches of a group over its items ordered by the kernel that their
-// cases take, one launch per kernel present.
-int batch_volume(const vcp_batch::Group &g, const vcp::StageCtl &ctl, hipStream_t s)
+// Volume launches of a group's cases from the given one on, over the items
+// ordered by the kernel that their cases take: one launch per kernel present.
+// Within a kernel the items stand in the order of the cases, so that those of
+// the last cases are its last ones.
+int batch_volume(const vcp_batch::Group &g, const vcp::StageCtl &ctl, hipStream_t s, size_t firstCase = 0)
 {
   vcp::BatchGroup v = g.view();
   v.work = g.dWorkV;
+  int n[vcp::kVolKinds] = {};
+  for (size_t ci = firstCase; ci < g.cases.size(); ++ci)
+    n[g.caseKind[ci]] += g.first[ci + 1] - g.first[ci];
   for (int k = 0; k < vcp::kVolKinds; ++k)
-    HIP_TRY(vcp::launch_batch_volume(v, k, ctl, g.kind[k], g.kind[k + 1] - g.kind[k], s));
+    HIP_TRY(vcp::launch_batch_volume(v, k, ctl, g.kind[k + 1] - n[k], n[k], s));
   return 0;
 }
 
@@ -176,9 +184,7 @@ int init_pass(vcp_batch *b)
     for (size_t ci = g.initFrom; ci < g.cases.size(); ++ci)
       HIP_TRY(vcp::launch_boundary(g.cases[ci]->dc, b->stream, false));
     HIP_TRY(vcp::launch_batch_faces(v, w0, nw, b->stream));
-    for (size_t ci = g.initFrom; ci < g.cases.size(); ++ci)
-      HIP_TRY(vcp::launch_batch_volume(v, vcp::volume_kind(g.cases[ci]->dc, g.nt), kResidualOnly, g.first[ci],
-                                       g.first[ci + 1] - g.first[ci], b->stream));
+    if (int rc = batch_volume(g, kResidualOnly, b->stream, (size_t) g.initFrom)) return rc;
     g.initFrom = -1;
   }
   return 0;
