@@ -157,17 +157,41 @@ int upload(vcp_batch *b)
   return 0;
 }
 
-// Volume launches of a group's cases from the given one on, over the items
-// ordered by the kernel that their cases take: one launch per kernel present.
-// Within a kernel the items stand in the order of the cases, so that those of
-// the last cases are its last ones.
+// The items of a group's cases from the given one on, in the list ordered by
+// the volume kernel that their cases take: n[k] of them up to g.kind[k + 1]
+// (within a kernel they stand in the order of the cases).
+void items_by_kind(const vcp_batch::Group &g, size_t firstCase, int (&n)[vcp::kVolKinds])
+{
+  for (int &x : n) x = 0;
+  for (size_t ci = firstCase; ci < g.cases.size(); ++ci)
+    n[g.caseKind[ci]] += g.first[ci + 1] - g.first[ci];
+}
+
+// Face launches of these cases: one, or in mixed precision one per volume
+// kernel present, which decides the precision of the flux lift.
+int batch_faces(const vcp_batch::Group &g, hipStream_t s, size_t firstCase = 0)
+{
+  if (g.cases.empty()) return 0;
+  vcp::BatchGroup v = g.view();
+  if (!g.mixed) {
+    HIP_TRY(vcp::launch_batch_faces(v, vcp::kVolWorkgroup, g.first[firstCase], g.nWork - g.first[firstCase], s));
+    return 0;
+  }
+  v.work = g.dWorkV;
+  int n[vcp::kVolKinds];
+  items_by_kind(g, firstCase, n);
+  for (int k = 0; k < vcp::kVolKinds; ++k)
+    HIP_TRY(vcp::launch_batch_faces(v, k, g.kind[k + 1] - n[k], n[k], s));
+  return 0;
+}
+
+// Volume launches of these cases: one per kernel present.
 int batch_volume(const vcp_batch::Group &g, const vcp::StageCtl &ctl, hipStream_t s, size_t firstCase = 0)
 {
   vcp::BatchGroup v = g.view();
   v.work = g.dWorkV;
-  int n[vcp::kVolKinds] = {};
-  for (size_t ci = firstCase; ci < g.cases.size(); ++ci)
-    n[g.caseKind[ci]] += g.first[ci + 1] - g.first[ci];
+  int n[vcp::kVolKinds];
+  items_by_kind(g, firstCase, n);
   for (int k = 0; k < vcp::kVolKinds; ++k)
     HIP_TRY(vcp::launch_batch_volume(v, k, ctl, g.kind[k + 1] - n[k], n[k], s));
   return 0;
@@ -179,11 +203,9 @@ int init_pass(vcp_batch *b)
 {
   for (vcp_batch::Group &g : b->groups) {
     if (g.initFrom < 0) continue;
-    const int w0 = g.first[g.initFrom], nw = g.nWork - w0;
-    const vcp::BatchGroup v = g.view();
     for (size_t ci = g.initFrom; ci < g.cases.size(); ++ci)
       HIP_TRY(vcp::launch_boundary(g.cases[ci]->dc, b->stream, false));
-    HIP_TRY(vcp::launch_batch_faces(v, w0, nw, b->stream));
+    if (int rc = batch_faces(g, b->stream, (size_t) g.initFrom)) return rc;
     if (int rc = batch_volume(g, kResidualOnly, b->stream, (size_t) g.initFrom)) return rc;
     g.initFrom = -1;
   }
@@ -201,7 +223,7 @@ int group_rk_step(const vcp_batch::Group &g, hipStream_t s)
   HIP_TRY(vcp::launch_batch_stage0(v, s));
   for (const vcp::StageCtl *ctl : {&kStage1, &kStage2, &kStage3}) {
     for (vcp_ctx *c : g.cases) HIP_TRY(vcp::launch_boundary(c->dc, s, false));
-    HIP_TRY(vcp::launch_batch_faces(v, 0, v.nWork, s));
+    if (int rc = batch_faces(g, s)) return rc;
     if (int rc = batch_volume(g, *ctl, s)) return rc;
   }
   return 0;
@@ -517,11 +539,10 @@ int vcp_batch_profile(vcp_batch *b, int reps, double *ms, int cap)
   for (int r = 0; r < reps; ++r)
     for (int gi = 0; gi < ng; ++gi) {
       const vcp_batch::Group &g = b->groups[gi];
-      const vcp::BatchGroup v = g.view();
       hipEvent_t *ev = &es.ev[3 * ((size_t) r * ng + gi)];
       HIP_TRY(hipEventRecord(ev[0], b->stream));
       for (vcp_ctx *c : g.cases) HIP_TRY(vcp::launch_boundary(c->dc, b->stream, false));
-      HIP_TRY(vcp::launch_batch_faces(v, 0, v.nWork, b->stream));
+      if ((rc = batch_faces(g, b->stream))) return rc;
       HIP_TRY(hipEventRecord(ev[1], b->stream));
       if ((rc = batch_volume(g, probe, b->stream))) return rc;
       HIP_TRY(hipEventRecord(ev[2], b->stream));

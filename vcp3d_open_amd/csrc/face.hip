@@ -17,6 +17,7 @@ template <int K, int M, typename T = double>
 struct FaceOps {
   EvenOdd<K, M, T> a;          // phi_q(r_p) and phi'_q(r_p), even-odd form
   EvenOddD<K, M, T> d;
+  EvenOdd<K, M, double> ad;    // phi_q(r_p) for the wide lift of the float form
   T A[M * K], D[M * K];        // the same, row-major (p, q)
   T F[4][K];                   // phi(-1), phi(+1), phi'(-1), phi'(+1)
   double w[M];                 // 1D Gauss weights
@@ -57,7 +58,7 @@ struct FaceArgs {
 // (6, 8) 16^3 194 / 133, (7, 9) 14^3 232 / 214; mixed (3, 4) 71 / 34,
 // (5, 7) 498 / 437. With the odd pitches and two waves per face at M = 9 below,
 // then: (6, 8) 16^3 130 / 106, (7, 9) 11^3 98 / 68, the others within 3 %.
-template <int K, int M, typename T = double>
+template <int K, int M, typename T, typename TL>
 struct FaceSmem {
   // faces per wave and lanes per face: the pointwise fluxes are half of the
   // instructions, and the M^2 points of one face leave most of a wave idle at
@@ -76,13 +77,15 @@ struct FaceSmem {
   // lines fall into different banks (at (6, 8) more than half of the LDS cycles
   // were conflicts, and the LDS 80 % busy)
   static constexpr int KP = K | 1, MP = M | 1, NP = M * MP;
-  static constexpr int kB = 2 * 2 * 5 * K * KP, kT1 = 13 * K * MP, kT = 2 * kT1, kP = 17 * NP;
-  static constexpr int kY = 13 * M * KP;
+  // in units of T; the flux and its first lift stage in TL
+  static constexpr int W = (int) (sizeof(TL) / sizeof(T));
+  static constexpr int kB = 2 * 2 * 5 * K * KP, kT1 = 13 * K * MP, kT = 2 * kT1, kP = (5 * W + 12) * NP;
+  static constexpr int kY = (5 * W + 8) * M * KP;
   // Y behind the fluxes, over T's end, where that lets one more face into a
   // CU's LDS and the face is large ((6, 8) 16^3: 110 us, 114 in a region of its
   // own); at (5, 7) the thirteenth face makes the launch slower (32^3: 554
   // against 542 us)
-  static constexpr int kOffY = M > 7 ? kP : cmax(cmax(kB, kT), kP);
+  static constexpr int kOffY = M > 7 ? kP : (cmax(cmax(kB, kT), kP) + W - 1) / W * W;
   static constexpr int kX = cmax(cmax(kB, kT), kOffY + kY);
   static constexpr int kBytes = (int) sizeof(T) * (2 * M * K + 4 * K + NF * kX) + 8 * (M * M + 1 + NF * 82);
   // waves per SIMD to compile for: three when 12 waves fit a CU's 160 KB
@@ -94,7 +97,7 @@ struct FaceSmem {
   struct Face {
     double Cm[2][4][9];            // metric of points 1..4 (bug)
     double Mean[2][5];             // float form: mode 0 of both elements
-    T X[kX];
+    alignas(8) T X[kX];
   } f[NF];
 };
 
@@ -104,10 +107,17 @@ struct FaceSmem {
 // arithmetic. T: the type of the contractions (double, or float for the
 // mixed-precision form, where the traces carry the variation about each
 // element's mean, added back at the points in double, and the pointwise
-// fluxes stay in double). SGS: the case has a subgrid scale model (a
+// fluxes stay in double). TL: the type in which the flux is lifted: T, or
+// double in the float form beside the column volume kernel, whose planes are in
+// double too. A residual is the difference of large interior and face terms,
+// and the flux and the operator rounded to float in one of them only leave a
+// pattern of their own in every element: after 20 steps of a 16^3 (5, 7) case
+// the density is off from the FP64 form's by 2.2e-8 with both in float, 6.0e-8
+// with the planes alone in double, 2.2e-9 with both (launch over the faces
+// 382 / 401 us at 32^3). SGS: the case has a subgrid scale model (a
 // separate instantiation: its eddy-viscosity code raises the register peak).
-template <int K, int M, int DIR, bool BUG, bool BATCH, typename T, bool SGS>
-__device__ __forceinline__ void face_body(const FaceArgs<K, M, T> &args, const CaseDev a, FaceSmem<K, M, T> &sm,
+template <int K, int M, int DIR, bool BUG, bool BATCH, typename T, typename TL, bool SGS>
+__device__ __forceinline__ void face_body(const FaceArgs<K, M, T> &args, const CaseDev a, FaceSmem<K, M, T, TL> &sm,
                                           int e, bool live)
 {
 #define VCP_FOPS (args.op)
@@ -118,7 +128,8 @@ __device__ __forceinline__ void face_body(const FaceArgs<K, M, T> &args, const C
   if (!__any(live)) return;
   if (L < 0) L = e;
   constexpr int ND = K * K * K, N2 = M * M;
-  using S = FaceSmem<K, M, T>;
+  using S = FaceSmem<K, M, T, TL>;
+  constexpr bool kWide = sizeof(TL) > sizeof(T);
   constexpr int G = S::G, NT = S::NT, KP = S::KP, MP = S::MP, NP = S::NP;
   constexpr int SB = 5 * K * KP;              // one plane of B
   // strides of the (normal, fast, slow) axes in the [k][j][i] DOF layout
@@ -133,7 +144,8 @@ __device__ __forceinline__ void face_body(const FaceArgs<K, M, T> &args, const C
   typename S::Face &sf = sm.f[lane / G];
   T *B = sf.X;                                // [side][value|deriv][5][K][KP]
   T *Tb = sf.X;                               // [side][A|D|N][5, 4, 4][K][MP]
-  T *sFlux = sf.X, *sFC = sf.X + 5 * NP;      // flux [5][M][MP], Cartesian sym [x|y|z][4][M][MP] of variables 1..4
+  TL *sFlux = (TL *) sf.X;                    // flux [5][M][MP]
+  T *sFC = sf.X + 5 * S::W * NP;              // Cartesian sym [x|y|z][4][M][MP] of variables 1..4
   // operators in LDS: read as wave-uniform LDS operands in the contractions
   // (as kernel arguments they would not fit the scalar registers)
   for (int i = lane; i < M * K; i += NT) { sA[i] = VCP_FOPS.A[i]; sD[i] = VCP_FOPS.D[i]; }
@@ -316,7 +328,7 @@ __device__ __forceinline__ void face_body(const FaceArgs<K, M, T> &args, const C
     const int mp = sp * MP + fp;
 #pragma unroll
     for (int v = 0; v < 5; ++v) {
-      sFlux[v * NP + mp] = T(fl[v]);
+      sFlux[v * NP + mp] = TL(fl[v]);
       if (v > 0) {
         sFC[(v - 1) * NP + mp] = T(FX[v]); sFC[(3 + v) * NP + mp] = T(FY[v]); sFC[(7 + v) * NP + mp] = T(FZ[v]);
       }
@@ -349,13 +361,41 @@ __device__ __forceinline__ void face_body(const FaceArgs<K, M, T> &args, const C
   // slot of that side: the value plane (A of the first, D of the slow slot)
   // and the normal-derivative plane (A of the normal slot) [0|1][v][slow]
   // [fast]; the volume kernel applies the face vectors.
+  // A of the wide lift stays in scalar registers over both sides from K = 4 on
+  // (32^3 (5, 7): 415 us, 432 with it loaded in each stage; at (3, 4) 36.5 / 36.1)
+  constexpr bool kKeep = kWide && K >= 4;
+  EvenOdd<K, M, TL> AL;
+  if constexpr (kKeep) AL = scalar_op<K, M, TL>(&ops()->ad);
+  auto wide_modes = [&](auto op, const TL (&x)[M], TL (&u)[K]) {
+    if constexpr (kKeep) to_modes(AL, x, u);
+    else to_modes(scalar_op<K, M, TL>(&op->ad), x, u);
+  };
+  // u += the derivative operator's transpose on x
+  auto add_derivs = [&](auto op, const T (&x)[M], TL (&u)[K]) {
+    T z[K];
+#pragma unroll
+    for (int n = 0; n < K; ++n) z[n] = 0;
+    add_modes(scalar_op<K, M, T>(&op->d), x, z);
+#pragma unroll
+    for (int n = 0; n < K; ++n) u[n] += TL(z[n]);
+  };
+  // a symmetrising slot alone, in T
+  auto slot_modes = [&](const EvenOdd<K, M, T> &A, const TL (&x)[M], TL (&u)[K]) {
+    T y[M], z[K];
+#pragma unroll
+    for (int p = 0; p < M; ++p) y[p] = T(x[p]);
+    to_modes(A, y, z);
+#pragma unroll
+    for (int n = 0; n < K; ++n) u[n] = TL(z[n]);
+  };
   constexpr bool kShare = S::NF == 1 && 9 * M <= G;
   static_assert(4 * K <= G || S::NF == 1, "the derivative plane's lines in one pass");
 #pragma unroll
   for (int side = 0; side < 2; ++side) {
-    const T sign = side ? T(1) : T(-1);
+    const TL sign = side ? TL(1) : TL(-1);
     double *out = a.faceRes + ((size_t) (side ? L : e) * 6 + 2 * DIR + side) * 10 * K * K;
-    T *Y0 = sf.X + S::kOffY, *YS = Y0 + 5 * M * KP, *YN = YS + 4 * M * KP;
+    TL *Y0 = (TL *) (sf.X + S::kOffY);
+    T *YS = sf.X + S::kOffY + 5 * S::W * M * KP, *YN = YS + 4 * M * KP;
     // Cartesian symmetrising flux mapped to this side's parametric slot P
     auto coef = [&](int v, int m, int P, int x) {
       return BUG ? sf.Cm[side][v][3 * P + x] : g[(side ? 4 + 3 * P + x : 13 + 3 * P + x) * N2 + m];
@@ -369,7 +409,8 @@ __device__ __forceinline__ void face_body(const FaceArgs<K, M, T> &args, const C
       if constexpr (BUG)
 #pragma unroll
         for (int x = 0; x < 3; ++x) { cb[x] = coef(vc, 0, P0, x); ca[x] = coef(vc, 0, PS, x); }
-      T xa[M], xb[M];
+      TL xa[M];
+      T xb[M];
 #pragma unroll
       for (int q = 0; q < M; ++q) {
         const int m = sp * M + q, mp = sp * MP + q;
@@ -379,25 +420,36 @@ __device__ __forceinline__ void face_body(const FaceArgs<K, M, T> &args, const C
           for (int x = 0; x < 3; ++x) { cb[x] = coef(vc, m, P0, x); ca[x] = coef(vc, m, PS, x); }
         xb[q] = !isSecond && v == 0 ? T(0) : T(fx * cb[0] + fy * cb[1] + fz * cb[2]);
         if (!second) xa[q] = sign * sFlux[v * NP + mp];
-        else if (!first) xa[q] = T(fx * ca[0] + fy * ca[1] + fz * ca[2]);
-        else xa[q] = isSecond ? T(fx * ca[0] + fy * ca[1] + fz * ca[2]) : sign * sFlux[v * NP + mp];
+        else if (!first) xa[q] = TL(fx * ca[0] + fy * ca[1] + fz * ca[2]);
+        else xa[q] = isSecond ? TL(fx * ca[0] + fy * ca[1] + fz * ca[2]) : sign * sFlux[v * NP + mp];
       }
       const auto op = ops();
-      const EvenOdd<K, M, T> A = scalar_op<K, M, T>(&op->a);
-      T u[K], w[K], z[K];
-      to_modes(A, xa, u);
-      if (second) to_modes(A, xb, w);
+      TL u[K], z[K];
+      T w[K];
+      if constexpr (kWide) {
+        if (first) wide_modes(op, xa, u);
+        if (second) {
+          const EvenOdd<K, M, T> A = scalar_op<K, M, T>(&op->a);
+          to_modes(A, xb, w);
+          if (!first) slot_modes(A, xa, u);
+        }
+      } else {
+        const EvenOdd<K, M, T> A = scalar_op<K, M, T>(&op->a);
+        to_modes(A, xa, u);
+        if (second) to_modes(A, xb, w);
+      }
       if (first) {
 #pragma unroll
         for (int n = 0; n < K; ++n) z[n] = u[n];
-        add_modes(scalar_op<K, M, T>(&op->d), xb, z);
+        if constexpr (kWide) add_derivs(op, xb, z);
+        else add_modes(scalar_op<K, M, T>(&op->d), xb, z);
         if (!isSecond)
 #pragma unroll
           for (int n = 0; n < K; ++n) Y0[idx * KP + n] = z[n];
       }
       if (second && isSecond)
 #pragma unroll
-        for (int n = 0; n < K; ++n) { YS[idx * KP + n] = u[n]; YN[idx * KP + n] = w[n]; }
+        for (int n = 0; n < K; ++n) { YS[idx * KP + n] = T(u[n]); YN[idx * KP + n] = w[n]; }
     };
     if constexpr (kShare) {
       if (tid < 9 * M) lines(tid, true, true, tid >= 5 * M);
@@ -413,15 +465,30 @@ __device__ __forceinline__ void face_body(const FaceArgs<K, M, T> &args, const C
     // slow-axis lines [0, 5 K) of the value plane, [5 K, 9 K) of the derivative plane
     auto planes = [&](int item, bool first, bool deriv) {
       const int idx = deriv ? item - 5 * K : item, v = deriv ? 1 + idx / K : idx / K, f = idx % K;
-      const T *ya = deriv ? YN + (v - 1) * M * KP + f : Y0 + v * M * KP + f;
+      const TL *y0 = Y0 + v * M * KP + f;
+      const T *yn = YN + (v - 1) * M * KP + f, *ya = deriv ? yn : (const T *) y0;
       const T *yb = YS + (v > 0 ? v - 1 : 0) * M * KP + f;
       const bool slow = !deriv && v > 0;
-      T xa[M], xb[M], u[K];
+      TL xa[M], u[K];
+      T xb[M];
 #pragma unroll
-      for (int q = 0; q < M; ++q) { xa[q] = ya[q * KP]; xb[q] = first && slow ? yb[q * KP] : T(0); }
+      for (int q = 0; q < M; ++q) {
+        if constexpr (kWide) xa[q] = deriv ? TL(yn[q * KP]) : y0[q * KP];
+        else xa[q] = ya[q * KP];
+        xb[q] = first && slow ? yb[q * KP] : T(0);
+      }
       const auto op = ops();
-      to_modes(scalar_op<K, M, T>(&op->a), xa, u);
-      if (first) add_modes(scalar_op<K, M, T>(&op->d), xb, u);
+      if constexpr (kWide) {
+        if (first) {
+          wide_modes(op, xa, u);
+          add_derivs(op, xb, u);
+        } else {
+          slot_modes(scalar_op<K, M, T>(&op->a), xa, u);
+        }
+      } else {
+        to_modes(scalar_op<K, M, T>(&op->a), xa, u);
+        if (first) add_modes(scalar_op<K, M, T>(&op->d), xb, u);
+      }
       if (!live) return;
       double *o = out + (deriv ? 5 * K * K : 0) + v * K * K + f;
 #pragma unroll
@@ -450,14 +517,14 @@ __device__ __forceinline__ void face_body(const FaceArgs<K, M, T> &args, const C
 // pointer: a by-value copy indexed at run time would go to scratch. The SGS
 // form is compiled for two waves per SIMD, where its eddy-viscosity code fits
 // the registers without spilling.
-template <int K, int M, bool BUG, bool BATCH, typename T, bool SGS>
-__global__ __launch_bounds__((FaceSmem<K, M, T>::NT), (SGS ? cmin(2, FaceSmem<K, M, T>::kWaves) : FaceSmem<K, M, T>::kWaves))
+template <int K, int M, bool BUG, bool BATCH, typename T, typename TL, bool SGS>
+__global__ __launch_bounds__((FaceSmem<K, M, T, TL>::NT), (SGS ? cmin(2, FaceSmem<K, M, T, TL>::kWaves) : FaceSmem<K, M, T, TL>::kWaves))
 void face_kernel(FaceArgs<K, M, T> a_)
 {
-  __shared__ FaceSmem<K, M, T> sm;
+  __shared__ FaceSmem<K, M, T, TL> sm;
   (void) a_;
   const FaceArgs<K, M, T> &a = *(const FaceArgs<K, M, T> *) __builtin_amdgcn_kernarg_segment_ptr();
-  using S = FaceSmem<K, M, T>;
+  using S = FaceSmem<K, M, T, TL>;
   const int sub = threadIdx.x / S::G, item = blockIdx.x * S::NF + sub;
   bool live = S::NF == 1 || item < a.n;
   CaseDev c;
@@ -472,9 +539,9 @@ void face_kernel(FaceArgs<K, M, T> a_)
     c = a.c;
     e = live ? item : 0;
   }
-  if (blockIdx.y == 0) face_body<K, M, 0, BUG, BATCH, T, SGS>(a, c, sm, e, live);
-  else if (blockIdx.y == 1) face_body<K, M, 1, BUG, BATCH, T, SGS>(a, c, sm, e, live);
-  else face_body<K, M, 2, BUG, BATCH, T, SGS>(a, c, sm, e, live);
+  if (blockIdx.y == 0) face_body<K, M, 0, BUG, BATCH, T, TL, SGS>(a, c, sm, e, live);
+  else if (blockIdx.y == 1) face_body<K, M, 1, BUG, BATCH, T, TL, SGS>(a, c, sm, e, live);
+  else face_body<K, M, 2, BUG, BATCH, T, TL, SGS>(a, c, sm, e, live);
 }
 
 template <int K, int M, typename T>
@@ -482,6 +549,7 @@ void fill_face_ops(const DeviceCase &dc, FaceOps<K, M, T> &op)
 {
   fill_even_odd(dc.opA, op.a);
   fill_even_odd(dc.opD, op.d);
+  fill_even_odd(dc.opA, op.ad);
   for (int i = 0; i < M * K; ++i) { op.A[i] = T(dc.opA[i]); op.D[i] = T(dc.opD[i]); }
   for (int q = 0; q < K; ++q)
     for (int t = 0; t < 4; ++t) op.F[t][q] = T(dc.opF[t][q]);
@@ -489,55 +557,56 @@ void fill_face_ops(const DeviceCase &dc, FaceOps<K, M, T> &op)
   op.c03 = dc.opC0[0] * dc.opC0[0] * dc.opC0[0];
 }
 
-template <int K, int M, bool BATCH, typename T, bool SGS>
+template <int K, int M, bool BATCH, typename T, typename TL, bool SGS>
 void launch_face_kernel(bool bug, int n, FaceArgs<K, M, T> &a, hipStream_t s)
 {
-  constexpr int NF = FaceSmem<K, M, T>::NF;
+  using S = FaceSmem<K, M, T, TL>;
+  const dim3 grid((n + S::NF - 1) / S::NF, 3), block(S::NT);
   a.n = n;
-  if (bug)
-    hipLaunchKernelGGL((face_kernel<K, M, true, BATCH, T, SGS>), dim3((n + NF - 1) / NF, 3), dim3(FaceSmem<K, M, T>::NT), 0, s, a);
-  else
-    hipLaunchKernelGGL((face_kernel<K, M, false, BATCH, T, SGS>), dim3((n + NF - 1) / NF, 3), dim3(FaceSmem<K, M, T>::NT), 0, s, a);
+  if (bug) hipLaunchKernelGGL((face_kernel<K, M, true, BATCH, T, TL, SGS>), grid, block, 0, s, a);
+  else hipLaunchKernelGGL((face_kernel<K, M, false, BATCH, T, TL, SGS>), grid, block, 0, s, a);
 }
 
-template <int K, int M, typename T>
-hipError_t faces_impl_t(const DeviceCase &dc, hipStream_t s)
+template <int K, int M, typename T, typename TL>
+hipError_t faces_impl(const DeviceCase &dc, hipStream_t s)
 {
   FaceArgs<K, M, T> a{};
   a.c = case_dev(dc);
   fill_face_ops(dc, a.op);
-  if (dc.sgs) launch_face_kernel<K, M, false, T, true>(dc.bug_compat, dc.nElem, a, s);
-  else launch_face_kernel<K, M, false, T, false>(dc.bug_compat, dc.nElem, a, s);
+  if (dc.sgs) launch_face_kernel<K, M, false, T, TL, true>(dc.bug_compat, dc.nElem, a, s);
+  else launch_face_kernel<K, M, false, T, TL, false>(dc.bug_compat, dc.nElem, a, s);
   return hipGetLastError();
 }
 
-template <int K, int M, typename T>
-hipError_t batch_faces_impl_t(const BatchGroup &g, int w0, int nw, hipStream_t s)
+template <int K, int M, typename T, typename TL>
+hipError_t batch_faces_impl(const BatchGroup &g, int w0, int nw, hipStream_t s)
 {
   FaceArgs<K, M, T> a{};
   a.cases = g.cases; a.work = g.work; a.w0 = w0;
   fill_face_ops(*g.proto, a.op);
-  if (g.proto->sgs) launch_face_kernel<K, M, true, T, true>(g.proto->bug_compat, nw, a, s);
-  else launch_face_kernel<K, M, true, T, false>(g.proto->bug_compat, nw, a, s);
+  if (g.proto->sgs) launch_face_kernel<K, M, true, T, TL, true>(g.proto->bug_compat, nw, a, s);
+  else launch_face_kernel<K, M, true, T, TL, false>(g.proto->bug_compat, nw, a, s);
   return hipGetLastError();
 }
 
 }  // namespace
 
 template <int K, int M>
-hipError_t faces(const DeviceCase &dc, hipStream_t s)
+hipError_t faces(const DeviceCase &dc, bool wide, hipStream_t s)
 {
-  return dc.mixed ? faces_impl_t<K, M, float>(dc, s) : faces_impl_t<K, M, double>(dc, s);
+  if (!dc.mixed) return faces_impl<K, M, double, double>(dc, s);
+  return wide ? faces_impl<K, M, float, double>(dc, s) : faces_impl<K, M, float, float>(dc, s);
 }
 
 template <int K, int M>
-hipError_t batch_faces(const BatchGroup &g, int w0, int nw, hipStream_t s)
+hipError_t batch_faces(const BatchGroup &g, bool wide, int w0, int nw, hipStream_t s)
 {
-  return g.proto->mixed ? batch_faces_impl_t<K, M, float>(g, w0, nw, s)
-                        : batch_faces_impl_t<K, M, double>(g, w0, nw, s);
+  if (!g.proto->mixed) return batch_faces_impl<K, M, double, double>(g, w0, nw, s);
+  return wide ? batch_faces_impl<K, M, float, double>(g, w0, nw, s)
+              : batch_faces_impl<K, M, float, float>(g, w0, nw, s);
 }
 
-template hipError_t faces<VCP_SHAPE_K, VCP_SHAPE_M>(const DeviceCase &, hipStream_t);
-template hipError_t batch_faces<VCP_SHAPE_K, VCP_SHAPE_M>(const BatchGroup &, int, int, hipStream_t);
+template hipError_t faces<VCP_SHAPE_K, VCP_SHAPE_M>(const DeviceCase &, bool, hipStream_t);
+template hipError_t batch_faces<VCP_SHAPE_K, VCP_SHAPE_M>(const BatchGroup &, bool, int, int, hipStream_t);
 
 }  // namespace vcp

@@ -1221,7 +1221,8 @@ int workgroup_tile(int K, int M, int nt)
 
 hipError_t launch_faces(const DeviceCase &dc, hipStream_t s)
 {
-#define X(k, m) if (dc.K == k && dc.M == m) return faces<k, m>(dc, s);
+  const bool wide = volume_kind(dc, dc.nt) != kVolWorkgroup;
+#define X(k, m) if (dc.K == k && dc.M == m) return faces<k, m>(dc, wide, s);
   VCP_PAIRS(X)
 #undef X
   return hipErrorInvalidValue;
@@ -1368,11 +1369,11 @@ hipError_t launch_stage0(const DeviceCase &dc, const double *dt, hipStream_t s)
   return hipGetLastError();
 }
 
-hipError_t launch_batch_faces(const BatchGroup &g, int w0, int nw, hipStream_t s)
+hipError_t launch_batch_faces(const BatchGroup &g, int kind, int w0, int nw, hipStream_t s)
 {
   if (nw <= 0) return hipSuccess;
   const DeviceCase &p = *g.proto;
-#define X(k, m) if (p.K == k && p.M == m) return batch_faces<k, m>(g, w0, nw, s);
+#define X(k, m) if (p.K == k && p.M == m) return batch_faces<k, m>(g, kind != kVolWorkgroup, w0, nw, s);
   VCP_PAIRS(X)
 #undef X
   return hipErrorInvalidValue;

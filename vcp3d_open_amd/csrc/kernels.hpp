@@ -178,13 +178,14 @@ hipError_t launch_faces(const DeviceCase &dc, hipStream_t s);
 // with monitor, also the wall forces into scal[kScalForce ..]
 hipError_t launch_boundary(const DeviceCase &dc, hipStream_t s, bool monitor = false);
 hipError_t launch_volume(const DeviceCase &dc, const StageCtl &ctl, hipStream_t s);
-// per supported pair: the faces (face.hip), the volume kernel with one
+// per supported pair: the faces (face.hip; wide: the float form's flux lift in
+// double, as beside the column volume kernel), the volume kernel with one
 // workgroup per element (volume_workgroup.hip; nt: its size) and the one with
 // one thread per column of points (volume.hip)
 template <int K, int M>
-hipError_t faces(const DeviceCase &dc, hipStream_t s);
+hipError_t faces(const DeviceCase &dc, bool wide, hipStream_t s);
 template <int K, int M>
-hipError_t batch_faces(const BatchGroup &g, int w0, int nw, hipStream_t s);
+hipError_t batch_faces(const BatchGroup &g, bool wide, int w0, int nw, hipStream_t s);
 template <int K, int M>
 hipError_t volume_workgroup(const DeviceCase &dc, int nt, const StageCtl &ctl, hipStream_t s);
 template <int K, int M>
@@ -220,8 +221,8 @@ hipError_t launch_stage0(const DeviceCase &dc, const double *dt, hipStream_t s);
 
 // Batched launches over the work items [w0, w0 + nw) of a group (cases whose
 // kWordActive word is 0 are skipped).
-hipError_t launch_batch_faces(const BatchGroup &g, int w0, int nw, hipStream_t s);
-// kind: volume_kind of every item's case
+// kind: volume_kind of every item's case (for the faces in mixed precision alone)
+hipError_t launch_batch_faces(const BatchGroup &g, int kind, int w0, int nw, hipStream_t s);
 hipError_t launch_batch_volume(const BatchGroup &g, int kind, const StageCtl &ctl, int w0, int nw, hipStream_t s);
 // The volume kernel of a case with the given workgroup size (0: the default):
 // volume_kernel, or the column kernel (volume.hip) in its plain form or, for a
