@@ -723,8 +723,10 @@ void volume_cols_kernel(ColArgs<K, M, T> args_)
   }
 
   // ---------------- w J rho, velocity and p / rho at the thread's points, for
-  // the weighted dU/dV of the solve
-  T pr[HP][5];
+  // the weighted dU/dV of the solve; in the float form w J p and the matrix's
+  // last entry in place of p / rho, formed in double and rounded once
+  constexpr int NPR = kMixed ? 6 : 5;
+  T pr[HP][NPR];
   {
     double J[HP];
     T V[5][HP];
@@ -748,10 +750,18 @@ void volume_cols_kernel(ColArgs<K, M, T> args_)
       const EntState st = ent_state(Vp);
       // the middle plane of an odd M belongs to the first half
       const bool mine = H == 1 || M % 2 == 0 || p < HP - 1 || h == 0;
-      pr[p][0] = mine ? T(w2 * op->w[p] * J[p] * st.rho) : T(0);
-      pr[p][1] = T(st.u); pr[p][2] = T(st.v); pr[p][3] = T(st.w); pr[p][4] = T(st.r);
+      if constexpr (kMixed) {
+        const double wr = mine ? w2 * op->w[p] * J[p] * st.rho : 0.0, P = wr * st.r, Et = st.r * kInvGm1 + st.ek;
+        pr[p][0] = T(wr);
+        pr[p][4] = T(P);
+        pr[p][5] = T(wr * Et * Et + P * (Et + st.ek));
+      } else {
+        pr[p][0] = mine ? T(w2 * op->w[p] * J[p] * st.rho) : T(0);
+        pr[p][4] = T(st.r);
+      }
+      pr[p][1] = T(st.u); pr[p][2] = T(st.v); pr[p][3] = T(st.w);
 #pragma unroll
-      for (int l = 0; l < 5; ++l) asm volatile("" : "+v"(pr[p][l]));
+      for (int l = 0; l < NPR; ++l) asm volatile("" : "+v"(pr[p][l]));
       __builtin_amdgcn_sched_barrier(0);
     }
   }
@@ -877,22 +887,35 @@ void volume_cols_kernel(ColArgs<K, M, T> args_)
         // E = e / (gamma - 1) + ek the total energy per mass:
         //   y0 = rho (p0 + u.p + E p4),  y_i = u_i y0 + P (p_i + u_i p4),
         //   y4 = E y0 + P (u.p + (E + ek) p4)
+        // or with rho E and the last entry d: y4 = rho E p0 + (rho E + P) u.p + d p4
 #pragma unroll
         for (int p = 0; p < HP; ++p) {
           if constexpr (kTight)
 #pragma unroll
-            for (int l = 0; l < 5; ++l) asm volatile("" : "+v"(pr[p][l]));
-          const T wr = pr[p][0], u = pr[p][1], v = pr[p][2], w = pr[p][3], eh = pr[p][4];
+            for (int l = 0; l < NPR; ++l) asm volatile("" : "+v"(pr[p][l]));
+          const T wr = pr[p][0], u = pr[p][1], v = pr[p][2], w = pr[p][3];
           const T kin = T(0.5) * (u * u + v * v + w * w);
-          const T Et = eh * T(kInvGm1) + kin, P = wr * eh;
-          const T p4 = y[4][p];
-          const T up = u * y[1][p] + v * y[2][p] + w * y[3][p];
-          const T y0 = wr * (y[0][p] + up + Et * p4);
-          y[0][p] = y0;
-          y[1][p] = u * y0 + P * (y[1][p] + u * p4);
-          y[2][p] = v * y0 + P * (y[2][p] + v * p4);
-          y[3][p] = w * y0 + P * (y[3][p] + w * p4);
-          y[4][p] = Et * y0 + P * (up + (Et + kin) * p4);
+          if constexpr (kMixed) {
+            const T P = pr[p][4], d = pr[p][5], rE = P * T(kInvGm1) + wr * kin;
+            const T p4 = y[4][p], up = u * y[1][p] + v * y[2][p] + w * y[3][p];
+            const T y0 = wr * (y[0][p] + up) + rE * p4, yP = y0 + P * p4;
+            y[4][p] = rE * y[0][p] + (rE + P) * up + d * p4;
+            y[0][p] = y0;
+            y[1][p] = u * yP + P * y[1][p];
+            y[2][p] = v * yP + P * y[2][p];
+            y[3][p] = w * yP + P * y[3][p];
+          } else {
+            const T eh = pr[p][4];
+            const T Et = eh * T(kInvGm1) + kin, P = wr * eh;
+            const T p4 = y[4][p];
+            const T up = u * y[1][p] + v * y[2][p] + w * y[3][p];
+            const T y0 = wr * (y[0][p] + up + Et * p4);
+            y[0][p] = y0;
+            y[1][p] = u * y0 + P * (y[1][p] + u * p4);
+            y[2][p] = v * y0 + P * (y[2][p] + v * p4);
+            y[3][p] = w * y0 + P * (y[3][p] + w * p4);
+            y[4][p] = Et * y0 + P * (up + (Et + kin) * p4);
+          }
           if (p % 2) __builtin_amdgcn_sched_barrier(0);
         }
         if constexpr (H == 1) {
