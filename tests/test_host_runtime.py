@@ -115,3 +115,34 @@ elements = sorted(int(line.split()[-1]) for line in launches("volume"))
 assert elements == [27 + 64, (1331 + 1) // 2], launches("volume")
 assert len(launches("face")) == 1
 """)
+
+
+TGV, BOX = "TGVCase(n={})", "OpenBoxCase(n=({}, 8, 8), sponge_elems=2)"
+
+
+# elements, and whether they take the column kernel: both sides of each line
+@pytest.mark.parametrize("precision,p,case,size,columns", [
+    ("fp64", 3, TGV, 10, False), ("fp64", 3, TGV, 11, True), ("fp64", 4, TGV, 9, False), ("fp64", 4, TGV, 10, True),
+    ("fp64", 5, TGV, 3, True), ("fp64", 6, TGV, 6, False), ("fp64", 6, TGV, 7, True),
+    ("mixed", 3, TGV, 11, False), ("mixed", 3, TGV, 12, True), ("mixed", 4, TGV, 9, False), ("mixed", 4, TGV, 10, True),
+    ("mixed", 5, TGV, 9, False), ("mixed", 5, TGV, 10, True), ("mixed", 6, TGV, 8, False), ("mixed", 6, TGV, 9, True),
+    ("fp64", 3, BOX, 40, False), ("fp64", 3, BOX, 41, True), ("fp64", 4, BOX, 48, False), ("fp64", 4, BOX, 49, True),
+    ("mixed", 3, BOX, 48, False), ("mixed", 3, BOX, 49, True), ("mixed", 4, BOX, 24, False), ("mixed", 4, BOX, 25, True),
+    ("mixed", 5, BOX, 36, False), ("mixed", 5, BOX, 37, True)])
+def test_volume_kernel_by_element_count(host_runtime, precision, p, case, size, columns):
+    case = case.format(size)[:-1] + f", p={p})"
+    host_runtime(f"""
+case = {case}
+s = SolverClass(case, precision={precision!r})
+s.ReadRestartSolution(case.initial_conservative())
+if isinstance(case, OpenBoxCase):
+    s.SetDampingState(case.damping_primitive())
+rt.rt_clear()
+s.Residual(False)
+taken, = launches("volume")
+assert taken.startswith("volume_cols_kernel<") == {columns}, taken
+# in mixed precision the faces follow: their flux lifted in double beside the column kernel
+if {precision!r} == "mixed":
+    face, = launches("face_kernel")
+    assert ("float, double" in face) == {columns}, face
+""")

@@ -1183,19 +1183,30 @@ int default_volume_tile(int K, int M)
 
 // Without a given size, the column kernel where the case has enough elements
 // to fill the chip with it: one wave per element (or several elements per
-// wave) runs longer per element than a workgroup, and 256 CUs hold few of
-// them. Measured on one box, volume launch in us, workgroup / column kernel:
-//   (4, 5) 512 elements 32.3 / 39.5, 1000: 39.1 / 43.7, 1331: 48.3 / 46.7, 1728: 64 / 53
-//   (4, 6) 512: 36.7 / 41.4, 1000: 68 / 44
-//   (5, 7) 512: 43.7 / 59.3, 1000: 78 / 65, 1728: 100 / 75
-// (4, 6) and (5, 7) hold 768 workgroups at once; the next element costs a
-// second round. With two threads per column (K >= 6 in FP64) the column kernel
-// is ahead from the smallest cases on at (6, 8) (27 elements 76 / 68) and once
-// every CU has one at (7, 9) (216: 73 / 77, 512: 134 / 91); in the float form from
-// a few hundred ((6, 8) 512: 48 / 63, 1000: 87 / 69; (7, 9) 512: 76 / 75).
-// At (3, 4) it is ahead at every size, up to 4096 elements with the columns in
-// halves, when these still run all at once (workgroup / halves / whole:
-// 64 elements 30.0 / 26.0 / 31.7, 1000: 32.3 / 25.4 / 29.9, 4096: 72 / 40 / 43,
+// wave) runs longer per element than a workgroup, which is ahead as long as the
+// chip holds all workgroups at once (1280 or, in the float form, 1536 of them at
+// (4, 5), 768 at (4, 6), (5, 7) and in the float form (6, 8), 256 or 512 at (7, 9)).
+// Measured on one box, volume launch in us, workgroup / column kernel,
+// Taylor-Green cases:
+//   (4, 5) 512 elements 31.8 / 39.4, 1000: 38.6 / 43.5, 1331: 47.2 / 46.2, 1728: 63 / 52
+//   float  1000: 24.4 / 32.4, 1331: 28.0 / 33.1, 1728: 40.2 / 34.5
+//   (4, 6) 512: 36.0 / 40.7, 1000: 67 / 44;  float 512: 27.0 / 31.2, 1000: 36.2 / 33.7
+//   (5, 7) 512: 42.3 / 58.3, 729: 51.5 / 61.0, 1000: 76 / 63, 1728: 99 / 74
+//   float  729: 36.6 / 46.0, 1000: 55 / 48
+//   (6, 8) 27: 76 / 68, 512: 84 / 70;  float 512: 46.4 / 62.1, 729: 56.9 / 64.6, 1000: 85 / 66
+//   (7, 9) 216: 72 / 77, 343: 133 / 92;  float 512: 76 / 74, 729: 113 / 77
+// (from (6, 8) on in FP64 a column has two threads). A case with boundaries
+// (a pulse, a wall layer) is uneven: the solve of most elements stops early, and
+// the launch lasts as long as its longest elements. The workgroup stays ahead up
+// to two rounds of them, four in FP64 and three in float at the high degrees:
+// open boxes with a pulse,
+//   (4, 5) 1280: 52 / 66, 1944: 61 / 66, 2916: 67 / 68;  float 1280: 33 / 43, 2916: 46 / 47
+//   (5, 7) 1152: 90 / 107, 1944: 102 / 100, 2916: 126 / 129, 5760: 211 / 192
+//   float  1152: 60 / 68, 1944: 74 / 65;  (6, 8) float 1152: 90 / 103, 1944: 110 / 124, 2916: 153 / 144
+//   (4, 6) 896: 69 / 62;  (7, 9) 384: 149 / 132
+// At (3, 4) the column kernel is ahead at every size, up to 4096 elements with
+// the columns in halves, when these still run all at once (workgroup / halves /
+// whole: 64 elements 30.0 / 26.0 / 31.7, 1000: 32.3 / 25.4 / 29.9, 4096: 72 / 40 / 43,
 // 5832: 85 / 57 / 49; float 64: 22.8 / 18.3 / 23.1, 4096: 38 / 29 / 32).
 int volume_kind(const DeviceCase &dc, int nt)
 {
@@ -1203,8 +1214,16 @@ int volume_kind(const DeviceCase &dc, int nt)
   const int cols = full ? kVolColsFull : kVolCols;
   if (nt) return nt == default_volume_tile(dc.K, dc.M) ? cols : kVolWorkgroup;
   if (dc.K == 3) return dc.nElem > 4096 ? cols : full ? kVolHalvesFull : kVolHalves;
-  const int least = dc.M == 5 ? 1280 : dc.K <= 5 ? 769 : dc.mixed ? 640 : dc.K == 6 ? 0 : 257;
-  return dc.nElem >= least ? cols : kVolWorkgroup;
+  // most elements for the workgroup kernel: [float][with boundaries]
+  struct Most {
+    int K, M, n[2][2];
+  };
+  static constexpr Most most[] = {{4, 5, {{1280, 2560}, {1536, 3072}}}, {4, 6, {{768, 768}, {768, 768}}},
+                                  {5, 7, {{768, 3072}, {768, 1536}}},   {6, 8, {{0, 0}, {768, 2304}}},
+                                  {7, 9, {{256, 256}, {512, 512}}}};
+  for (const Most &m : most)
+    if (m.K == dc.K && m.M == dc.M) return dc.nElem > m.n[dc.mixed != 0][dc.nBFace > 0] ? cols : kVolWorkgroup;
+  return kVolWorkgroup;
 }
 
 namespace {
