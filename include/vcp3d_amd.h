@@ -327,7 +327,10 @@ int vcp_batch_set_graph(vcp_batch *b, int enable);
 /* Volume workgroup size of the group (nDOFs1D, nInt1D) (see vcp_set_tile). */
 int vcp_batch_set_tile(vcp_batch *b, int n_dofs_1d, int n_int_1d, int nt);
 /* Groups: info[g][7] = {nDOFs1D, nInt1D, bug_compat, cases, work items,
-   volume workgroup size, precision}; returns the number of groups. */
+   volume workgroup size, precision}; returns the number of groups. The size is
+   the given one (vcp_batch_set_tile), or the one that all cases of the group
+   take by themselves; 0 where they differ or take the columns in halves of
+   nDOFs1D = 3, which no size names. */
 int vcp_batch_groups(vcp_batch *b, int *info, int cap);
 /* Measurement: mean milliseconds of `reps` residual evaluations per group,
    ms[2 g] boundary + face kernels, ms[2 g + 1] volume kernel (cap: entries

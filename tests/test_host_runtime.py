@@ -146,3 +146,25 @@ if {precision!r} == "mixed":
     face, = launches("face_kernel")
     assert ("float, double" in face) == {columns}, face
 """)
+
+
+def test_groups_report_the_kernel_that_runs(host_runtime):
+    """A group's volume size is the one that runs: the given one, the one that
+    all its cases take by themselves, or 0 where none names it (cases that differ,
+    the split columns of P = 2)."""
+    host_runtime("""
+small, large, low = solver(n=3, p=4), solver(n=10, p=4), solver(n=3, p=2)
+batch = Batch()
+size = lambda K: next(g["nt"] for g in batch.groups() if g["K"] == K)
+batch.add(small); batch.add(low)
+assert size(5) == 256 and size(3) == 0
+batch.add(large)
+assert size(5) == 0
+batch.remove(small)
+assert size(5) == 64
+batch.set_tile(5, 7, 512)
+assert size(5) == 512
+batch.set_tile(5, 7, 0)
+batch.step(1)
+assert [line for line in launches("volume") if "<5, 7, 512" in line] == []
+""")

@@ -513,7 +513,13 @@ int vcp_batch_groups(vcp_batch *b, int *info, int cap)
     if (n < cap) {
       int *o = info + 7 * n;
       o[0] = g.K; o[1] = g.M; o[2] = g.bug; o[3] = (int) g.cases.size(); o[4] = g.nWork;
-      o[5] = g.nt ? g.nt : vcp::default_volume_tile(g.K, g.M);
+      // the given size, or the one that all cases take by themselves
+      o[5] = g.nt;
+      if (!g.nt && !g.cases.empty()) {
+        o[5] = vcp::volume_tile(g.caseKind[0], g.K, g.M);
+        for (int k : g.caseKind)
+          if (vcp::volume_tile(k, g.K, g.M) != o[5]) o[5] = 0;
+      }
       o[6] = g.mixed;
     }
     ++n;

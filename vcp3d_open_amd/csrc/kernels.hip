@@ -1175,7 +1175,7 @@ int volume_tiles(int K, int M, int out[4])
   return n;
 }
 
-int default_volume_tile(int K, int M)
+int column_tile(int K, int M)
 {
   int t[4];
   return volume_tiles(K, M, t) > 0 ? t[0] : 0;
@@ -1212,7 +1212,7 @@ int volume_kind(const DeviceCase &dc, int nt)
 {
   const bool full = dc.sgs != kSgsNone || dc.nSponge > 0 || dc.fbodyOn;
   const int cols = full ? kVolColsFull : kVolCols;
-  if (nt) return nt == default_volume_tile(dc.K, dc.M) ? cols : kVolWorkgroup;
+  if (nt) return nt == column_tile(dc.K, dc.M) ? cols : kVolWorkgroup;
   if (dc.K == 3) return dc.nElem > 4096 ? cols : full ? kVolHalvesFull : kVolHalves;
   // most elements for the workgroup kernel: [float][with boundaries]
   struct Most {
@@ -1237,6 +1237,12 @@ int workgroup_tile(int K, int M, int nt)
   return nt;
 }
 }  // namespace
+
+int volume_tile(int kind, int K, int M)
+{
+  if (kind == kVolWorkgroup) return workgroup_tile(K, M, 0);
+  return kind == kVolCols || kind == kVolColsFull ? column_tile(K, M) : 0;
+}
 
 hipError_t launch_faces(const DeviceCase &dc, hipStream_t s)
 {

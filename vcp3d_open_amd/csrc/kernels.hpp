@@ -170,9 +170,10 @@ struct BatchGroup {
   X(7, 9, 512)
 
 bool supported_pair(int K, int M);
-// Volume workgroup sizes available for (K, M); the first is the default.
+// Volume workgroup sizes available for (K, M): the column kernel's name first,
+// then volume_kernel's sizes.
 int volume_tiles(int K, int M, int out[4]);
-int default_volume_tile(int K, int M);
+int column_tile(int K, int M);
 hipError_t launch_faces(const DeviceCase &dc, hipStream_t s);
 // boundary-averaged Mach number partial sums, then the PC-NSCBC faces
 // with monitor, also the wall forces into scal[kScalForce ..]
@@ -230,6 +231,8 @@ hipError_t launch_batch_volume(const BatchGroup &g, int kind, const StageCtl &ct
 // K = 3 for cases of few elements the column kernel with the columns in halves.
 enum : int { kVolWorkgroup = 0, kVolCols = 1, kVolColsFull = 2, kVolHalves = 3, kVolHalvesFull = 4, kVolKinds = 5 };
 int volume_kind(const DeviceCase &dc, int nt);
+// the size that names this kernel, 0 for the columns in halves, which have none
+int volume_tile(int kind, int K, int M);
 // per-element time steps, then per case: the minimum, the synchronization-step
 // clipping into scal[kScalDt], and the step counters; a case with error flags
 // or no steps left is deactivated instead

@@ -350,7 +350,9 @@ class SolverClass:
 
 
 def volume_tiles(K: int, M: int) -> list:
-    """Volume workgroup sizes available for (K, M), the default first."""
+    """Volume workgroup sizes available for (K, M): the column kernel's, then
+    those of one workgroup per element. The default (size 0) is chosen per case
+    among them by its element count."""
     L = load_library()
     out = np.zeros(4, dtype=np.int32)
     n = L.vcp_volume_tiles(K, M, out)
