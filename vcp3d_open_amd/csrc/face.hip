@@ -336,7 +336,7 @@ __device__ __forceinline__ void face_body(const FaceArgs<K, M, T> &args, const C
   };
   if constexpr (NT > 64) {
     if (atPoint) traces();
-    __syncthreads();
+    group_sync<NT>();
     if (atPoint) fluxes();
   } else if (atPoint) {
     traces();
@@ -348,7 +348,7 @@ __device__ __forceinline__ void face_body(const FaceArgs<K, M, T> &args, const C
     evMax = lanes_reduce<G, true>(evMax);
     if constexpr (NT > 64) {
       if (tid == 64) sm.EvMax = evMax;
-      __syncthreads();
+      group_sync<NT>();
       evMax = fmax(evMax, sm.EvMax);
     }
     if (tid == 0 && live) a.eddyPart[a.nElem + 3 * e + DIR] = evMax;

@@ -103,7 +103,7 @@ __device__ __forceinline__ void group_reduce(double (&v)[NV], double *red, int &
     if ((threadIdx.x & 63) == 0)
 #pragma unroll
       for (int q = 0; q < NV; ++q) buf[wid * NV + q] = v[q];
-    __syncthreads();
+    group_sync<G>();
 #pragma unroll
     for (int q = 0; q < NV; ++q) {
       double s = buf[q];
