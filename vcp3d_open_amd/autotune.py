@@ -1,18 +1,19 @@
 """Volume workgroup-size autotuner for batched stepping.
 
-The volume kernel of each (nDOFs1D, nInt1D) shape is compiled for several
-workgroup sizes (threads per element; vcp_volume_tiles lists them). Which one
-is fastest depends on the shape: a small element (K = 3) leaves most of a
-256-thread workgroup idle in its pencil stages, while a large one (K = 7) needs
-512 threads to hold one DOF per thread. The tuner times every size of every
-group of a batch on the batch's own cases (vcp_batch_profile: residual
-evaluations that store nothing, HIP events around each launch) and keeps the
-fastest. Sizes give results equal to rounding (the mass-matrix solve groups
-its partial sums differently), and a given size gives identical results
-every run.
+The volume kernel of each (nDOFs1D, nInt1D) shape comes in several forms
+(vcp_volume_tiles lists them): one thread per column of points, and one
+workgroup per element of several sizes. By itself (size 0) each case takes the
+one that is fastest at its element count and precision. The tuner times size 0
+and every form of every group of a batch on the batch's own cases
+(vcp_batch_profile: residual evaluations that store nothing, HIP events around
+each launch) and keeps the fastest, size 0 among equals. A form other than 0
+holds for all cases of its shape, whatever their size. Forms give results equal
+to rounding (the mass-matrix solve groups its partial sums differently), and a
+given form gives identical results every run.
 
-The choice is recorded per device architecture in tiles_<arch>.json beside
-this file: {"K,M": {"nt": best, "ms": {nt: volume ms per launch}}}.
+The choice can be recorded per device architecture in tiles_<arch>.json beside
+this file: {"K,M": {"nt": best, "ms": {nt: volume ms per launch}}}. Without a
+record every shape takes size 0.
 """
 from __future__ import annotations
 
@@ -43,9 +44,10 @@ def load_tiles(arch: str = "gfx950") -> dict:
 
 
 def tune(batch: Batch, reps: int = 5) -> dict:
-    """Times every volume workgroup size of every (K, M) shape of the batch
-    (summed over the groups of that shape); sets the fastest on the batch and
-    returns {(K, M): {"nt": best, "ms": {nt: volume ms per launch}}}."""
+    """Times the choice by element count (0) and every volume workgroup size
+    for every (K, M) shape of the batch (summed over the groups of that shape);
+    sets the fastest on the batch and returns
+    {(K, M): {"nt": best, "ms": {nt: volume ms per launch}}}."""
     shapes = []
     for g in batch.groups():
         if (g["K"], g["M"]) not in shapes:
@@ -53,7 +55,7 @@ def tune(batch: Batch, reps: int = 5) -> dict:
     result = {}
     for K, M in shapes:
         times = {}
-        for nt in volume_tiles(K, M):
+        for nt in [0] + volume_tiles(K, M):
             batch.set_tile(K, M, nt)
             prof = batch.profile(reps)
             times[nt] = sum(ms_vol for g, (_, ms_vol) in zip(batch.groups(), prof)
