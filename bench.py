@@ -38,9 +38,56 @@ PEAK_FP64_TFLOPS = 78.6   # MI355X dense FP64 (vector and matrix)
 PEAK_HBM_GBS = 8000.0
 
 
-def volume_kernel_flops(K: int, M: int, cg_iters: float) -> float:
-    """Algorithmic FLOPs per element of the fused volume + mass-matrix kernel
-    (2 per multiply-add; sum-factorised contraction counts, 350 flops per
+def to_points_flops(K: int, M: int) -> int:
+    """One line of K modes to M points with the even-odd operator: even modes at
+    the points of the first half and the middle, odd modes at those of the
+    first half, their sum and difference."""
+    he, ho, ke, ko = (M + 1) // 2, M // 2, (K + 1) // 2, K // 2
+    return he * (2 * ke - 1) + ho * (2 * ko - 1) + 2 * ho
+
+
+def to_modes_flops(K: int, M: int) -> int:
+    """Its transpose: sums and differences of the mirrored points, then both parts."""
+    he, ho, ke, ko = (M + 1) // 2, M // 2, (K + 1) // 2, K // 2
+    return 2 * ho + ke * (2 * he - 1) + ko * (2 * ho - 1)
+
+
+def line_derivative_flops(M: int) -> int:
+    """Derivative along a line of M point values, or its transpose, with the
+    centro-antisymmetric operator in two halves."""
+    h, odd = M // 2, M % 2
+    return 2 * h + (2 * h - 1) * odd + h * (2 * (2 * h - 1) + 2 * odd + 2)
+
+
+def column_kernel_flops(K: int, M: int, cg_iters: float, halves: bool = False) -> float:
+    """FLOPs per element that the column volume kernel carries out (2 per
+    multiply-add; even-odd transforms, line derivatives in place of the dense
+    derivative operators; 350 flops per integration point for gradients and
+    fluxes, 70 for the point state of the solve). halves: two threads per column,
+    whose contractions along the column are dense."""
+    col_p = M * (2 * K - 1) if halves else to_points_flops(K, M)
+    col_m = K * (2 * M - 1) if halves else to_modes_flops(K, M)
+    lines = 5 * (K * K + K * M)                  # along i and j, all variables
+    to_columns, to_modal = lines * to_points_flops(K, M), lines * to_modes_flops(K, M)
+    planes = M**3 * (5 * (4 * K - 4) + 350 + 5 * (4 * K - 1)) + 18 * M * M * line_derivative_flops(M)
+    point_state = 5 * M * M * col_p + 70 * M**3
+    gather = 120 * K**3                          # six faces x (value, derivative plane) x 5 variables
+    solve = to_columns + 5 * M * M * (col_p + col_m) + 37 * M**3 + to_modal + 74 * K**3
+    return to_columns + planes + point_state + to_modal + gather + cg_iters * solve
+
+
+def volume_flops(K: int, M: int, cg_iters: float, nt: int, mixed: bool = False) -> float:
+    """FLOPs per element of the volume kernel of size nt (0: per case, counted
+    as the column kernel)."""
+    from vcp3d_open_amd.solver import volume_tiles
+    if nt in volume_tiles(K, M)[1:]:
+        return workgroup_kernel_flops(K, M, cg_iters)
+    return column_kernel_flops(K, M, cg_iters, halves=K >= 6 and not mixed)
+
+
+def workgroup_kernel_flops(K: int, M: int, cg_iters: float) -> float:
+    """FLOPs per element of the volume kernel with one workgroup per element
+    (2 per multiply-add; dense sum-factorised contractions, 350 flops per
     integration point for the pointwise flux work)."""
     fwd = 5 * (2 * K**3 * M + 3 * K**2 * M**2 + 4 * K * M**3)
     bwd = 5 * (3 * K * M**3 + 3 * K**2 * M**2 + 2 * K**3 * M)
@@ -72,16 +119,30 @@ def measured_traffic(kernel: str):
 
 
 def face_kernel_flops(K: int, M: int) -> float:
-    """Algorithmic FLOPs per element-face (both traces, flux, both lifts to
-    the tangential coefficient planes); 700 flops per face point for the
-    Ismail-Roe + viscous + penalty work."""
-    trace = 2 * 5 * (2 * K**3 + 3 * K**2 * M + 4 * K * M**2)
-    lift = 2 * 5 * (4 * K * M**2 + 3 * K**2 * M)
-    return 2.0 * (trace + lift) + 700.0 * M**2
+    """FLOPs per element-face that the face kernel carries out (both traces,
+    flux, both lifts to the tangential coefficient planes; even-odd lines); 700
+    flops per face point for the Ismail-Roe + viscous + penalty work."""
+    eo_p, eo_m = to_points_flops(K, M), to_modes_flops(K, M)
+    normal = 2 * 5 * K * K * 2 * (2 * K - 1)
+    fast = 2 * 5 * K * 3 * eo_p
+    points = 2 * M * M * (5 * (2 * K - 1) + 4 * 3 * (2 * K - 1) + 4 * 18) + 700 * M * M
+    lift = 2 * ((9 * M + 4 * M) * eo_m + 5 * M * eo_m + 2 * 5 * 9 * M * M + (9 * K + 4 * K) * eo_m)
+    return float(normal + fast + points + lift)
 
 
 def face_kernel_bytes(K: int, M: int) -> float:
     return 8.0 * (2 * 5 * K**3 + 22 * M**2 + 2 * 10 * K**2 + 2)
+
+
+def volume_size(solver) -> int:
+    """The volume size that names the kernel this case runs."""
+    from vcp3d_open_amd.solver import Batch
+    batch = Batch()
+    batch.add(solver)
+    nt = batch.groups()[0]["nt"]
+    batch.remove(solver)
+    batch.close()
+    return nt
 
 
 def calib_copy(nbytes: int) -> int:
@@ -228,10 +289,10 @@ def bench_batch(args) -> int:
         per_group.append({"P": K - 1, "K": K, "M": M, "cases": g["cases"], "elements": g["work"],
                           "volume_threads": g["nt"], "ms_face_kernel": ms_face, "ms_volume_kernel": ms_vol,
                           "cg_iters_mean": cg,
-                          "volume_tflops": volume_kernel_flops(K, M, cg) * g["work"] / (ms_vol * 1e-3) / 1e12})
+                          "volume_tflops": volume_flops(K, M, cg, g["nt"], g["mixed"]) * g["work"] / (ms_vol * 1e-3) / 1e12})
     top = max(per_group, key=lambda x: x["ms_volume_kernel"])
     K, M = top["K"], top["M"]
-    flops = volume_kernel_flops(K, M, top["cg_iters_mean"]) * top["elements"]
+    flops = volume_flops(K, M, top["cg_iters_mean"], top["volume_threads"], args.precision == "mixed") * top["elements"]
     bytes_ = volume_kernel_bytes(K, M) * top["elements"]
     ms = top["ms_volume_kernel"]
     achieved = flops / (ms * 1e-3) / 1e12
@@ -445,7 +506,7 @@ def main() -> int:
     ap.add_argument("--seed", type=int, default=2024, help="batch: seed of the case draw")
     ap.add_argument("--cases", type=int, default=64, help="batch: number of cases; serve: number of requests")
     ap.add_argument("--autotune", action="store_true",
-                    help="batch: time every volume workgroup size per shape and record the table")
+                    help="batch: time every volume form per shape and record the table")
     ap.add_argument("--graph", action="store_true", help="batch: replay each RK step as a HIP graph")
     ap.add_argument("--precision", choices=["fp64", "mixed"], default="fp64",
                     help="arithmetic of the measured line: fp64 (default) or mixed (FP32 contractions and "
@@ -469,7 +530,7 @@ def main() -> int:
         return bench_interpolation(args)
 
     from vcp3d_open_amd.cases import OpenBoxCase, TGVCase
-    from vcp3d_open_amd.solver import SolverClass
+    from vcp3d_open_amd.solver import SolverClass, volume_tiles
 
     if args.workload == "openbox":
         case = OpenBoxCase(n=(48, 24, 24), p=4, rule=12, sponge_elems=8)
@@ -516,8 +577,9 @@ def main() -> int:
     rs_face, rs_vol = solver.profile_residual(args.profile_reps)
     K, M = case.p + 1, 7
     if ms_vol >= ms_face:
-        name, ms = "volume_cols_kernel<5, 7>", ms_vol
-        flops = volume_kernel_flops(K, M, cg_mean) * case.n_elems
+        nt = volume_size(solver)
+        name, ms = ("volume_cols_kernel<5, 7>" if nt == volume_tiles(K, M)[0] else f"volume_kernel<5, 7, {nt}>"), ms_vol
+        flops = volume_flops(K, M, cg_mean, nt, args.precision == "mixed") * case.n_elems
         bytes_ = volume_kernel_bytes(K, M, 2.0 / 3.0) * case.n_elems
     else:
         name, ms = "face_kernel<5, 7, BUG> (3 directions)", ms_face
