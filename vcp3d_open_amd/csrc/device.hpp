@@ -127,10 +127,13 @@ __device__ inline void ent2prim(const double V[5], double &rho, double &u, doubl
 }
 
 
-// 1 / x and 1 / sqrt(x) to rounding: the hardware approximation with its error
-// removed by Newton steps, without the scaling and exception steps of the IEEE
-// division and square root (fewer than half of their instructions). x <= 0,
-// infinite or not a number gives infinite or not-a-number, as these do.
+// 1 / x and 1 / sqrt(x) to about a unit in the last place: the hardware
+// approximation with its error removed by Newton steps, without the scaling and
+// exception steps of the IEEE division and square root (fewer than half of their
+// instructions). recip holds for x of either sign whose reciprocal is a normal
+// number; 0 and infinity give not-a-number, where the division gives infinity
+// and 0. rsqrt_exact holds for normal x > 0; 0, negative and infinite x give
+// not-a-number.
 __device__ __forceinline__ double recip(double x)
 {
   double y = __builtin_amdgcn_rcp(x);

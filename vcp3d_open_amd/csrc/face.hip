@@ -51,13 +51,15 @@ struct FaceArgs {
 // not memory. The line contractions use the even-odd operators, the lift
 // fills the wave (9 M lines per side), the pointwise fluxes take five
 // reciprocals and roots instead of twenty divisions and square roots, and two
-// or four faces share a wave at M = 5 and 4: 1520 vector instructions per
-// face instead of 2070 at (5, 7). Measured, launch over the three directions
-// of a Taylor-Green case before / after, us: (3, 4) 18^3 72 / 43,
-// (4, 5) 16^3 68 / 48, (4, 6) 14^3 54 / 46, (5, 7) 32^3 612 / 530,
-// (6, 8) 16^3 194 / 133, (7, 9) 14^3 232 / 214; mixed (3, 4) 71 / 34,
-// (5, 7) 498 / 437. With the odd pitches and two waves per face at M = 9 below,
-// then: (6, 8) 16^3 130 / 106, (7, 9) 11^3 98 / 68, the others within 3 %.
+// or four faces share a wave at M = 5 and 4: 1570 vector instructions per
+// face instead of 2070 at (5, 7). Measured on one box, launch over the three
+// directions of a Taylor-Green case, with dense lines and one face per wave /
+// as it is, us: (3, 4) 18^3 68 / 38, (4, 5) 16^3 65 / 44, (4, 6) 14^3 51 / 42,
+// (5, 7) 32^3 577 / 473, (6, 8) 16^3 187 / 103, (7, 9) 14^3 226 / 125; float
+// form, with the flux lifted in float / in double: (3, 4) 36 / 36, (4, 5) 36 / 35,
+// (4, 6) 39 / 40, (5, 7) 385 / 401, (6, 8) 74 / 86, (7, 9) 107 / 116. The odd
+// pitches and, at M = 9, the two waves per face are a fifth of it at (6, 8) and a third
+// at (7, 9) (130 / 106 at 16^3, 98 / 68 at 11^3).
 template <int K, int M, typename T, typename TL>
 struct FaceSmem {
   // faces per wave and lanes per face: the pointwise fluxes are half of the

@@ -1,14 +1,17 @@
-// gfx950 kernels of the VCP3D explicit DG residual and SSP-RK3 stage (FP64).
+// gfx950 kernels of the VCP3D explicit DG residual and SSP-RK3 stage beside the
+// three that are compiled per shape, and the launches of all of them.
 //
-//   face_kernel          interior (incl. periodic) faces: traces of both
-//                        elements, Ismail-Roe + viscous + penalty +
+// Per shape, in sources of their own:
+//   face_kernel          (face.hip) interior (incl. periodic) faces: traces of
+//                        both elements, Ismail-Roe + viscous + penalty +
 //                        symmetrising fluxes, lifted to both elements into
 //                        per-element face slots (no atomics)
-//   volume_kernel        volume residual, gather of the six face slots,
-//                        per-element entropy mass-matrix PCG, optional
-//                        in-place RK stage update, one workgroup per element:
-//                        the form of small cases; large ones take the column
-//                        kernel of volume.hip
+//   volume_cols_kernel   (volume.hip) volume residual, gather of the six face
+//                        slots, per-element entropy mass-matrix PCG, optional
+//                        in-place RK stage update, one thread per column of points
+//   volume_kernel        (volume_workgroup.hip) the same with one workgroup per
+//                        element: the form of small cases
+// Here:
 //   mach_kernel          boundary-averaged Mach number partial sums (NSCBC)
 //   nscbc_kernel         PC-NSCBC boundary faces: characteristic boundary
 //                        state, polynomial-correction reconstruction, flux

@@ -122,8 +122,7 @@ __device__ __forceinline__ void group_reduce(double (&v)[NV], double *red, int &
 // from the last one down, by the second. The whole column in one thread needs a
 // third fewer instructions (the even-odd transforms), but 10 M values and the
 // solve's vectors must fit 256 registers: beyond K = 5 in FP64 they spill ((6, 8)
-// at 16^3: 0.415 ms whole, 0.335 ms halved; (5, 7) at 32^3: 1.04 ms whole, 1.38 ms
-// halved). At K = 3 cases of few elements take halves too (volume_kind): they
+// at 16^3 halved: 0.81 of the whole column's time; (5, 7) at 32^3: 1.32 of it). At K = 3 cases of few elements take halves too (volume_kind): they
 // fill twice as many waves, each with half of the column's serial work.
 template <int K, typename T>
 constexpr int kColHalves = K >= 6 && sizeof(T) == 8 ? 2 : 1;
@@ -136,16 +135,17 @@ struct ColShape {
   static constexpr int G = H * LH;                       // threads per element
   static constexpr int NE = G < 64 ? 64 / G : 1;         // elements per workgroup
   static constexpr int NT = G < 64 ? 64 : G;
-  // waves per SIMD to compile for: at three (168 registers) every shape spills
-  // and runs slower ((4, 5) at 16^3 0.164 against 0.081 ms)
+  // waves per SIMD to compile for: at three (168 registers) every shape whose
+  // LDS lets three run spills, between 4 registers ((4, 6), float) and 240
+  // ((7, 9)); measured at (4, 5), where 135 spill: 16^3 0.164 against 0.081 ms
   static constexpr int WAVES = 2;
   static constexpr int HP = H == 1 ? M : (M + 1) / 2;    // planes of a thread (the second half of an odd M: one less)
   static constexpr bool kInWave = H == 2 && LH < 64;     // the halves share a wave
   // pitches, odd so that lanes a pitch apart fall into different banks
   static constexpr int KP = K | 1, MP = M | 1, NP = N2 | 1;
   // the planes' lines of one variable, PL apart: at M = 8 a value more than
-  // their length, without which they collide in the banks (16^3 358 / 353 us;
-  // at M = 4 and 6 the gaps cost more, 59 / 57 and 98 / 97 us)
+  // their length, without which they collide in the banks (1.4 % of the launch
+  // at (6, 8); at M = 4 and 6 the gaps cost more, 3 and 1 %)
   static constexpr int PL = M % 8 ? M : M + 1, LP = (M * PL) | 1;
   // half-transformed lines of one (variable, k): K lines without a gap at
   // K >= 6 (lines a pitch apart throughout: with a gap of one the 64 lanes of
@@ -276,11 +276,12 @@ __device__ __forceinline__ void columns_to_modes(const EvenOdd<K, M, T> &A, T *X
 // latency at two waves per SIMD (it issues 45-60 % of the time), which the
 // registers set: scratch costs most of all (20 spilled registers cost 30 % at
 // (5, 7)), so the scheduling barriers below keep the phases apart.
-// Measured, workgroup / column form, volume launch of a Taylor-Green case:
-//   FP64   (3, 4) 18^3 95 / 55 us    (4, 5) 16^3 127 / 82    (4, 6) 14^3 150 / 96
-//          (5, 7) 32^3 1535 / 1042   (6, 8) 16^3 620 / 335   (7, 9) 14^3 720 / 458
-//   float  (3, 4) 60 / 38   (4, 5) 69 / 47   (4, 6) 95 / 52   (5, 7) 1075 / 737
-//          (6, 8) 265 / 209   (7, 9) 385 / 233
+// Measured on one box, workgroup / column form, volume launch of a residual of a
+// curvilinear Taylor-Green case:
+//   FP64   (3, 4) 18^3 87 / 47 us    (4, 5) 16^3 109 / 66    (4, 6) 14^3 129 / 81
+//          (5, 7) 32^3 1405 / 937   (6, 8) 16^3 540 / 272   (7, 9) 14^3 641 / 408
+//   float  (3, 4) 56 / 33   (4, 5) 63 / 43   (4, 6) 87 / 60   (5, 7) 1021 / 676
+//          (6, 8) 229 / 182   (7, 9) 365 / 207
 template <int K, int M, bool BATCH, bool FULL, typename T, int HALVES>
 __global__ __launch_bounds__((ColShape<K, M, T, HALVES>::NT), (ColShape<K, M, T, HALVES>::WAVES))
 void volume_cols_kernel(ColArgs<K, M, T> args_)
@@ -562,11 +563,12 @@ void volume_cols_kernel(ColArgs<K, M, T> args_)
     }
   };
   // ---------------- sponge, matching-layer and body-force sources, in planes
-  // of their own ahead of the fluxes': beside the fluxes they spill 40
-  // registers in every element, of those outside the sponge too. Volume launch
-  // of the 48 x 24 x 24 open box at (5, 7), 8 of 48 element layers in the
-  // sponge: 888 us beside the fluxes, 718 us here; 18^3 (3, 4) with WALE,
-  // which these sources spilled as well: 57 / 53 us.
+  // of their own ahead of the fluxes': beside the fluxes they spilled 40
+  // registers in every element, of those outside the sponge too; here (4, 5)
+  // spills 2 (FP64) or 13 (24 in a batch), (7, 9) 4 or 10, the other shapes at
+  // most 3. Volume launch of the 48 x 24 x 24 open box at (5, 7), 8 of 48 element
+  // layers in the sponge: 888 us beside the fluxes, 718 us here; 18^3 (3, 4) with
+  // WALE, which these sources spilled as well: 57 / 53 us.
   if constexpr (FULL)
     if (sp >= 0 || a->bfBuf) {
 #pragma unroll 1
