@@ -281,7 +281,9 @@ int vcp_set_tile(vcp_ctx *ctx, int nt);
    volume kernels and the mass-matrix solve in FP32 (the solve stops at
    ||r||_inf < 1e-5 ||r0||_inf), while the state and its element means, the
    pointwise flux physics, the face-slot gather, the metric terms, the NSCBC
-   boundary kernels, the time step and the RK update stay in FP64.
+   boundary kernels, the time step and the RK update stay in FP64. With the
+   column volume kernel (vcp_set_tile) the fluxes are contracted and lifted in
+   FP64 too.
    VCP_PRECISION_FP64 (the default) is the reference's arithmetic. */
 enum { VCP_PRECISION_FP64 = 0, VCP_PRECISION_MIXED = 1 };
 int vcp_set_precision(vcp_ctx *ctx, int mode);
@@ -291,7 +293,8 @@ int vcp_volume_tiles(int n_dofs_1d, int n_int_1d, int out[4]);
    Many independent cases stepped together, with no counterpart in the
    reference (one SolverClass per case, SolverClass.hpp:40-124): the cases
    are grouped by (nDOFs1D, nInt1D, bug_compat, precision), and each kernel of an RK
-   stage is one launch per group over a work list of (case, element) items.
+   stage is one launch per group over a work list of (case, element) items (one
+   per volume kernel where a group's cases take different ones).
    Each case keeps its own time step and the synchronization-step clipping of
    ExecuteTimeSynchronizationStep (SolverClass.cpp:2356-2365) on the device:
    a case advanced n RK steps by the batch holds the state that n RK steps of

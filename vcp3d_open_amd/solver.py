@@ -345,7 +345,8 @@ class SolverClass:
         self.precision = precision
 
     def set_tile(self, nt: int) -> None:
-        """Volume workgroup size (threads per element; 0: the default)."""
+        """Volume workgroup size (one of volume_tiles; 0: chosen by the element
+        count)."""
         self._check(self._L.vcp_set_tile(self.h, int(nt)))
 
 
